@@ -695,11 +695,12 @@ namespace vkhip {
     }
 
     // conv_halo_kernel: 3x3, stride 1 or 2 (both axes), pad 1, dilation 1, output (H - 1)/S + 1,
-    // Cin a multiple of the stage's 16*KK channels (odd input widths take the ODD variant).
+    // Cin a multiple of the stage's 16*KK channels, or any on the RC tiles (odd input widths take the ODD variant).
     static bool halo_shape_ok(const vkhip_conv_desc *d, const TileCfg &t) {
         const int S = d->SH;
         return d->group == 1 && d->KH == 3 && d->KW == 3 && (S == 1 || S == 2) && d->SW == S && d->PT == 1 && d->PL == 1 &&
-               d->DH == 1 && d->DW == 1 && d->OH == (d->H - 1) / S + 1 && d->OW == (d->W - 1) / S + 1 && d->Cin % (16 * t.KK) == 0;
+               d->DH == 1 && d->DW == 1 && d->OH == (d->H - 1) / S + 1 && d->OW == (d->W - 1) / S + 1 &&
+               (t.RC || d->Cin % (16 * t.KK) == 0);
     }
 
     // 1 KB copy chunks per channel slot of the largest input band any workgroup of a halo tile
@@ -796,9 +797,9 @@ namespace vkhip {
             g.nsteps = ceil_div((int64_t) d->KH * d->KW * thin_cinb(g.Cinb) * 4, 32);
             g.Kp     = g.nsteps * 32;
         }
-        if (t.kind == 3) { // 9 taps x Cin, stages of 16*KK channels (all 9 taps each)
-            g.Kp     = 9 * (int64_t) d->Cin;
-            g.nsteps = d->Cin / (16 * t.KK);
+        if (t.kind == 3) { // 9 taps x Cin, stages of 16*KK channels (all 9 taps each), the last one zero padded
+            g.nsteps = ceil_div(d->Cin, 16 * t.KK);
+            g.Kp     = 9 * g.nsteps * 16 * t.KK;
         }
         g.m_tiles = ceil_div(g.Coutb * 4, t.BM);
         g.Coutp   = g.m_tiles * t.BM;

@@ -1,4 +1,4 @@
-// Tile instantiations of conv_halo_kernel (tiles 17-20, 26, 27, 32-35: 3x3 with the input band staged once).
+// Tile instantiations of conv_halo_kernel (tiles 17-20, 26, 27, 32-35, 50-53: 3x3 with the input band staged once).
 #include "conv_kernels.h"
 
 namespace vkhip {
@@ -16,12 +16,16 @@ namespace vkhip {
     GemmKernelFn halo_tile_kernel(int tile, int nbi) {
         switch (tile) {
             case 17: return pick_halo<2, 2, 2, 2, 1, 3, 1, 2, 3, 4>(nbi);
+            case 50: // any channel count: the same kernels, the slots past the last block copied as zeros
             case 18: return pick_halo<2, 2, 1, 4, 1, 2, 1, 2, 3, 4, 5, 6, 8, 10, 12, 15>(nbi);
             case 19: return pick_halo<2, 4, 2, 2, 1, 2, 2, 3, 4, 5, 6, 8, 10>(nbi);
             case 20: return pick_halo<2, 1, 1, 4, 1, 1, 1, 2, 3, 4, 5, 6, 8, 10, 12, 16>(nbi);
+            case 51:
             case 26: return pick_halo<2, 1, 1, 4, 1, 2, 1, 2, 3, 4, 5, 6, 8>(nbi);
             case 27: return pick_halo<2, 2, 1, 4, 1, 1, 2, 4, 6, 8, 10, 12, 15>(nbi);
+            case 52:
             case 32: return pick_halo<1, 2, 1, 4, 1, 2, 1, 2, 3, 4, 5, 6, 8, 10, 12, 15>(nbi);
+            case 53:
             case 33: return pick_halo<1, 1, 1, 4, 1, 2, 1, 2, 3, 4, 5, 6, 8>(nbi);
             case 34: return pick_halo<1, 2, 1, 4, 1, 1, 2, 4, 6, 8, 10, 12, 16>(nbi);
             case 35: return pick_halo<1, 1, 1, 4, 1, 1, 2, 4, 6, 8, 10>(nbi);

@@ -1500,7 +1500,8 @@ namespace vkhip {
     }
 
     // ------------------------------------------------------------------ 3x3 halo-tile GEMM kernel
-    // Direct 3x3 pad-1 convolution, stride 1 or 2 (Cin a multiple of 16*KK, even input width W),
+    // Direct 3x3 pad-1 convolution, stride 1 or 2 (the last K stage of a channel count that is not a
+    // multiple of 16*KK is filled with zero slots),
     // that reads each input pixel once per workgroup instead of once per tap: the workgroup's BN
     // consecutive output pixels (row-major over n, oy, ox, free to cross image boundaries) need a
     // band of input rows (rows S*oy - 1 .. S*oy + 1 of each output row oy);
@@ -1607,9 +1608,11 @@ namespace vkhip {
             for (int r = 0; r < NBW; ++r) {
                 const int c  = r * NW + wave;
                 const int sl = c / NBI;
-                const unsigned vo = bsrc[c % NBI]; // (a local: the host pass rejects the array element as a builtin operand)
+                // slots past the last channel block (a channel count that fills no whole stage): zeros
+                const bool     in = ks * SLOTS + sl < a.Cinb; // wave-uniform
+                const unsigned vo = in ? bsrc[c % NBI] : kInvalid;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void *) (dst + BOFF + sl * SS + (c % NBI) * 1024),
-                                                         16, vo, (unsigned) (ks * SLOTS + sl) * hw8, 0, 0);
+                                                         16, vo, in ? (unsigned) (ks * SLOTS + sl) * hw8 : 0u, 0, 0);
             }
         };
 
@@ -2126,7 +2129,11 @@ namespace vkhip {
     // kind 2: conv_dma_kernel (A and B via LDS DMA; dense B only: 1x1 s1 with an even pixel count
     //         per image, Winograd GEMMs with an even tile count), 2x2 waves of (32FM) x (32FN).
     // kind 3: conv_halo_kernel (3x3 pad-1, stride 1 or 2: input band staged once in LDS for all 9
-    //         taps), KK 16-channel K steps per LDS stage.
+    //         taps), KK 16-channel K steps per LDS stage. RC = b: the kernel and geometry of tile b,
+    //         for any channel count (tile b keeps to multiples of 16*KK). Against the best gather tile
+    //         on counts that are not (us): 65 -> 341 at 35x17 b37 39.3 -> 23.7, 333 -> 47 at 15x57 b110
+    //         90.7 -> 45.5, 149 -> 46 at 69x18 b24 20.2 -> 11.3, 72 -> 72 at 28x28 b32 17.5 -> 9.9,
+    //         201 -> 71 stride 2 at 76x74 b3 19.9 -> 13.9: the gather reads each input pixel 9 times.
     // kind 4: conv_stem_kernel (3x3 or 7x7, stride 1 or 2, pad K/2, at most 4 input channels).
     // kind 5: conv_thin_kernel (3x3 pad 1 or 1x1, stride 1 or 2, at most 32 input channels and BM
     //         output channels, FM = BM / 16 fragments; weights in registers).
@@ -2134,7 +2141,7 @@ namespace vkhip {
     // workgroups, each walking a strided list of tiles.
     // LE (kind 2 only): the LDS-staged epilogue (gemm_epilogue_lds).
     struct TileCfg {
-        int BM, BN, WM, WN, kind, FM, FN, KK, PERS, LE;
+        int BM, BN, WM, WN, kind, FM, FN, KK, PERS, LE, RC;
     };
     static const TileCfg kTiles[] = {
         {128, 128, 2, 2, 0, 0, 0}, // 0
@@ -2187,10 +2194,14 @@ namespace vkhip {
         {64, 128, 2, 2, 2, 1, 2, 0, 0, 1},  // 47 tile 24 with the LDS-staged epilogue
         {128, 128, 2, 2, 2, 2, 2, 0, 0, 1}, // 48 tile 29 (3-stage ring) with the LDS-staged epilogue
         {64, 128, 2, 2, 2, 1, 2, 0, 0, 1},  // 49 tile 31 (4-stage ring) with the LDS-staged epilogue
+        {64, 256, 1, 4, 3, 2, 2, 1, 0, 0, 18}, // 50 tile 18 for any channel count
+        {64, 128, 1, 4, 3, 2, 1, 1, 0, 0, 26}, // 51 tile 26 for any channel count
+        {32, 256, 1, 4, 3, 1, 2, 1, 0, 0, 32}, // 52 tile 32 for any channel count
+        {32, 128, 1, 4, 3, 1, 1, 1, 0, 0, 33}, // 53 tile 33 for any channel count
     };
-    constexpr int kNumTiles = 50;
+    constexpr int kNumTiles = 54;
     constexpr int kHaloMaxNBI[kNumTiles] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 4, 15, 10, 16, 48, 48, 48, 0, 0, 8, 15, 0, 0, 0, 0, 15, 8, 16, 10,
-                                            0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                                            0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 15, 8, 15, 8};
 
     typedef void (*GemmKernelFn)(GemmArgs);
 
