@@ -178,7 +178,7 @@ typedef struct vkhip_conv_plan {
 
 /* Fill `plan` for `algo` (AUTO picks by shape heuristics). `tile` < 0 picks the default tile; for
  * a depthwise conv `tile` is the number of output rows per strip of the row-tiled kernel (4, 7 or
- * 14; 0 or < 0: chosen by shape). */
+ * 14; 0 or < 0: chosen by shape, the matrix-core kernel wherever its 8-pixel window holds the taps). */
 int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, int32_t ksplit, vkhip_conv_plan *plan);
 int vkhip_conv_tile_count(void);
 /* Name of the kernel family a plan launches (e.g. "conv_dma_kernel"; Winograd names its three

@@ -1,0 +1,86 @@
+"""The matrix-core depthwise kernel (dwconv_cols_kernel, plan tile 0) against the CPU oracle at the
+edges of its column split: planes narrower than a window, one column left over, row bands, odd
+widths, odd output rows at stride 2, pads above and beside K/2, ragged channels, every activation,
+residual and pool sums; and infinities, which may only reach the outputs whose window holds them.
+
+The kernel sums the same fp16 x fp16 products in fp32 as the oracle, in another order, and rounds
+once to fp16: bar max|d|/max|ref| <= 2e-2 and cosine >= 0.9999, as for every conv kernel here.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import vknn_amd as V
+from tests.gpu_helpers import check, conv_desc, from_device_nc4, gpu_conv, round_half, to_device_nc4
+from tests.oracle_lib import oracle_conv, parity
+
+pytestmark = pytest.mark.gpu
+
+
+def case(shape, k, s, pads, act, res):
+    r = np.random.default_rng(shape[1] * 7 + shape[2] + k + s)
+    x = round_half(r.standard_normal(shape))
+    w = round_half(r.standard_normal((shape[1], 1, k, k)) * 0.3)
+    b = (r.standard_normal(shape[1]) * 0.1).astype(np.float32)
+    d, ys = conv_desc(shape, w.shape, (s, s), pads, group=shape[1], act=act, has_res=int(res))
+    return x, w, b, d, ys, round_half(r.standard_normal(ys)) if res else None
+
+
+@pytest.mark.parametrize("k,s", [(3, 1), (3, 2), (5, 1), (5, 2)])
+@pytest.mark.parametrize("shape,act,res", [((1, 4, 1, 1), 0, False), ((1, 6, 2, 3), 1, True), ((3, 20, 7, 7), 4, False), ((2, 5, 15, 33), 5, True),
+                                           ((17, 8, 9, 14), 2, False), ((1, 16, 112, 112), 3, False), ((128, 12, 14, 14), 4, True)])
+def test_cols_against_oracle(gpu, shape, act, res, k, s):
+    p = k // 2
+    x, w, b, d, ys, rr = case(shape, k, s, (p,) * 4, act, res)
+    lo, hi = (-0.5, 0.7) if act == 3 else (0.0, 0.0)
+    got, plan, _ = gpu_conv(x, w, b, (s, s), (p,) * 4, group=shape[1], act=act, lo=lo, hi=hi, res=rr)
+    assert plan.algo == V.CONV_DEPTHWISE and plan.tile == 0
+    ref = oracle_conv(x, w, b, (s, s), (p,) * 4, group=shape[1], res=rr, act=act, lo=lo, hi=hi)
+    rel, cos = parity(got, ref)
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
+# pads (top, left, bottom, right); 5x5 stride 1 with an odd left pad does not fit the window: strip kernel
+@pytest.mark.parametrize("k,s,pads", [(3, 1, (0, 0, 0, 0)), (3, 2, (0, 0, 1, 1)), (3, 1, (2, 2, 2, 2)), (5, 2, (1, 1, 2, 2)), (5, 1, (1, 1, 1, 1)),
+                                      (5, 1, (0, 0, 4, 4)), (5, 1, (4, 4, 0, 0)), (3, 2, (3, 3, 3, 3))])
+def test_cols_pads(gpu, k, s, pads):
+    x, w, b, d, ys, _ = case((2, 10, 13, 18), k, s, pads, 0, False)
+    got, _, _ = gpu_conv(x, w, b, (s, s), pads, group=10)
+    rel, cos = parity(got, oracle_conv(x, w, b, (s, s), pads, group=10))
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
+@pytest.mark.parametrize("k,s", [(3, 1), (3, 2), (5, 1), (5, 2)])
+def test_cols_infinities_stay_in_their_window(gpu, k, s):
+    p = k // 2
+    x, w, b, d, ys, _ = case((2, 8, 17, 22), k, s, (p,) * 4, 0, False)
+    x[0, 2, 5, 7], x[1, 6, 0, 21], x[1, 1, 16, 0] = np.inf, -np.inf, np.nan
+    got, _, _ = gpu_conv(x, w, b, (s, s), (p,) * 4, group=8)
+    ref = oracle_conv(x, w, b, (s, s), (p,) * 4, group=8)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    inf, fin = np.isinf(ref), np.isfinite(ref)
+    assert inf.any() and np.array_equal(got[inf], ref[inf])
+    rel, cos = parity(got[fin], ref[fin])
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
+@pytest.mark.parametrize("shape,k,s", [((3, 22, 14, 14), 3, 1), ((4, 960, 7, 7), 5, 1), ((2, 12, 29, 31), 5, 2), ((1, 8, 40, 9), 3, 2)])
+def test_cols_pool_sums(gpu, shape, k, s):
+    """The parts of a plane add up to the sum of the stored fp16 outputs: fp32 sums of at most
+    H * W values each, so their relative error is below H * W * 2^-24 < 1e-4."""
+    lib, p = V.vkhip(), k // 2
+    x, w, b, d, ys, _ = case(shape, k, s, (p,) * 4, 4, False)
+    ref, plan, dref = gpu_conv(x, w, b, (s, s), (p,) * 4, group=shape[1], act=4)
+    blob = np.zeros(plan.weight_bytes, np.uint8)
+    check(lib.vkhip_conv_pack_weights(ctypes.byref(d), ctypes.byref(plan), w.ctypes.data, b.ctypes.data, blob.ctypes.data))
+    parts = lib.vkhip_conv_pool_parts(ctypes.byref(d), ctypes.byref(plan))
+    cb = (shape[1] + 3) // 4
+    dx, db = to_device_nc4(x), V.DeviceBuffer.from_array(blob)
+    dy, dp = V.DeviceBuffer(V.nc4_elems(*ys) * 2), V.DeviceBuffer(shape[0] * cb * parts * 16)
+    check(lib.vkhip_conv_forward_pooled(ctypes.byref(d), ctypes.byref(plan), dx.ptr, db.ptr, None, dy.ptr, dp.ptr, None))
+    check(lib.vkhip_stream_sync(None))
+    assert np.array_equal(from_device_nc4(dy, ys), ref)
+    got = dp.download(np.float32, shape[0] * cb * parts * 4).reshape(shape[0], cb, parts, 4).astype(np.float64).sum(2)
+    want = ref.astype(np.float64).sum((2, 3))
+    np.testing.assert_allclose(got.reshape(shape[0], -1)[:, :shape[1]], want, atol=1e-4 * np.abs(ref).sum((2, 3)).max())

@@ -176,19 +176,6 @@ namespace vkhip {
     // ------------------------------------------------------------------ depthwise
     // Thread = (n, cb, oy, OXT consecutive ox) of one 4-channel block; fp16 weights [Cb][KH][KW][4]
     // and bias [Cb*4]. Reference semantics: ConvCpu with group == C (conv.cpp:40-80).
-    struct DwArgs {
-        const uint2 *x;
-        const half4 *w;    // fp16 weights [Cb][KH][KW] x 4 channels
-        const float *bias;
-        const uint2 *res;
-        uint2       *y;
-        int          N, Cb, C, H, W, OH, OW, KH, KW, SH, SW, PT, PL, DH, DW;
-        int          act;
-        float        lo, hi;
-        int          has_res;
-        float4v     *pool; // dwconv_lds_kernel: per-(plane, row tile) sums of the stored outputs, or null
-    };
-
     template <int KH, int KW, int S, int OXT>
     __global__ __launch_bounds__(256) void dwconv_kernel(DwArgs a) {
         const int kh = KH > 0 ? KH : a.KH;
@@ -934,7 +921,7 @@ const char *vkhip_conv_plan_kernel(const vkhip_conv_plan *plan) {
     static const char *kinds[] = {"conv_gemm_kernel", "conv_bd_kernel", "conv_dma_kernel", "conv_halo_kernel", "conv_stem_kernel", "conv_thin_kernel"};
     if (!plan) return "?";
     if (plan->algo == VKHIP_CONV_GEMM && plan->tile >= 0 && plan->tile < kNumTiles && kTiles[plan->tile].PERS) return "conv_dma_persist_kernel";
-    if (plan->algo == VKHIP_CONV_DEPTHWISE) return "dwconv_lds_kernel";
+    if (plan->algo == VKHIP_CONV_DEPTHWISE) return plan->tile ? "dwconv_lds_kernel" : "dwconv_cols_kernel";
     if (plan->tile < 0 || plan->tile >= kNumTiles) return "?";
     if (plan->algo == VKHIP_CONV_WINOGRAD) return "wino_input_kernel+conv_gemm_kernel+wino_output_kernel";
     return kinds[kTiles[plan->tile].kind];
@@ -1207,6 +1194,8 @@ static int conv_forward_impl(const vkhip_conv_desc *d, const vkhip_conv_plan *pl
         a.act = d->act; a.lo = d->act_lo; a.hi = d->act_hi; a.has_res = d->has_res;
         a.pool = (float4v *) pool;
         bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
+        DwCols cols;
+        if (plan->tile == 0 && dw_cols_plan(d, cols)) return dw_cols_launch(a, cols, st);
         DwTile t;
         const int RT = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
         if (unit && d->KH == d->KW && (d->KH == 3 || d->KH == 5) && (d->SH == 1 || d->SH == 2) &&
@@ -1409,6 +1398,8 @@ int vkhip_conv_forward_view_res(const vkhip_conv_desc *d, const vkhip_conv_plan 
 
 int vkhip_conv_pool_parts(const vkhip_conv_desc *d, const vkhip_conv_plan *plan) {
     if (!d || !plan || plan->algo != VKHIP_CONV_DEPTHWISE || d->in_scale) return 0;
+    DwCols cols;
+    if (plan->tile == 0 && dw_cols_plan(d, cols)) return cols.NB * cols.parts;
     const bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
     const int  RT   = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
     DwTile     t;

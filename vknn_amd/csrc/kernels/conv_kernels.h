@@ -2234,4 +2234,28 @@ namespace vkhip {
     StemPoolFn stem_pool_kernel_for(int K, int cfg);
     GemmKernelFn stem_tile_kernel(int tile, int bmode, int nbi);
 
+    // ------------------------------------------------------------------ depthwise arguments
+    struct DwArgs {
+        const uint2 *x;
+        const half4 *w;    // fp16 weights [Cb][KH][KW] x 4 channels
+        const float *bias;
+        const uint2 *res;
+        uint2       *y;
+        int          N, Cb, C, H, W, OH, OW, KH, KW, SH, SW, PT, PL, DH, DW;
+        int          act;
+        float        lo, hi;
+        int          has_res;
+        float4v     *pool; // per-(plane, part) sums of the stored outputs (vkhip_conv_pool_parts per plane), or null
+    };
+    // Column split of dwconv_cols_kernel (dwconv_cols.hip).
+    struct DwCols {
+        int XB, NB, BR; // windows per row, row bands per plane, output rows per band
+        int groups;     // groups of 16 columns per channel block
+        int off;        // window pixel of tap 0 of output 0 (left pad rounded up to even, minus the pad)
+        int Q;          // columns per channel block: N * NB * XB
+        int parts;      // pool sums per (plane, band): the groups that its windows can lie in
+    };
+    bool dw_cols_plan(const vkhip_conv_desc *d, DwCols &t);
+    int  dw_cols_launch(const DwArgs &a, const DwCols &t, hipStream_t st);
+
 } // namespace vkhip
