@@ -299,7 +299,7 @@ namespace vknn {
                         if (!tok.empty()) skipTiles.insert(std::atoi(tok.c_str()));
                 }
                 for (int t = 0; t < ntiles; ++t)
-                    if (!skipTiles.count(t)) cands.push_back({VKHIP_CONV_GEMM, t, 0});
+                    if (!skipTiles.count(t) && (t < 50 || d.Cin % 16)) cands.push_back({VKHIP_CONV_GEMM, t, 0});
                 if (dw) // 0: the matrix-core kernel where it applies; else the strip kernel's rows per strip
                     // + 100 x strips per workgroup, 900: persistent plane groups (VKNN_HIP_DW_PIPE=0: one strip only)
                     for (int rt: {0, 4, 7, 14, 204, 207, 404, 407, 907, 914})
@@ -312,7 +312,8 @@ namespace vknn {
                 // with the big tiles) and the reduction is deep enough to split.
                 const int64_t kdepth = (int64_t) d.KH * d.KW * ((d.Cin + 3) / 4) * 4;
                 if (!dw && (pixels <= 4096 || base.algo == VKHIP_CONV_SPLITK || (pixels * (int64_t) d.Cout <= (int64_t) 512 * 128 * 256 && kdepth >= 512))) {
-                    for (int t: {3, 6, 1, 8, 10, 14, 16, 17, 18, 20, 26})
+                    // (the any-channel halo tiles only where the tiles they share their kernels with refuse)
+                    for (int t: d.Cin % 16 ? std::vector<int> {3, 8, 10, 14, 24, 28, 51, 53} : std::vector<int> {3, 10, 14, 16, 20, 24, 26, 28, 33})
                         for (int ks: {2, 3, 4, 8, 16})
                             for (int alg: {VKHIP_CONV_SPLITK, VKHIP_CONV_SPLITK_LAST}) cands.push_back({alg, t, ks});
                 }

@@ -849,6 +849,138 @@ namespace vkhip {
 
     static size_t align256(size_t v) { return (v + 255) & ~(size_t) 255; }
 
+    // ------------------------------------------------------------------ AUTO
+    // Predicted time (us) of a plan, a sum of what a launch costs, what its workgroups and K stages
+    // cost per CU, and what its tensors cost from memory. The coefficients were fitted (non-negative
+    // least squares on relative errors) to every such plan's measured time on 930 random 1x1 and 3x3
+    // layers: batch 1-128, 16-2048 channels, maps of 7-80 pixels, odd sizes among them.
+    //   1x1: 1, W, W S, S, MB, q S, q, part MB          3x3 (halo): 1, W, W S, S, MB, part MB, W S n, S n, q S, q
+    // W: workgroups per CU, S: K stages per split (64 values; 3x3: 16 channels), MB: activations read and
+    // written, part MB: fp32 partials, r: workgroups that share a CU's LDS, q: ceil(W / r), n: 1 KB copies
+    // per channel slot of a 3x3's input band.
+    struct AutoCost {
+        int   tile, split;
+        float c[10];
+    };
+    static const AutoCost kAuto1x1[] = {
+        {24, 0, {2.336f, 0.4389f, 0.116f, 0, 0.06709f, 0.3707f, 1.55f, 0}},
+        {31, 0, {2.321f, 0.5927f, 0, 0, 0.06199f, 0.3693f, 1.614f, 0}},
+        {37, 0, {2.799f, 0, 0.07057f, 0, 0.08288f, 0.3014f, 2.698f, 0}},
+        {39, 0, {3.548f, 0, 0.02961f, 0, 0.08668f, 0.2645f, 1.297f, 0}},
+        {41, 0, {3.315f, 0.1826f, 0.04376f, 0, 0.1231f, 0.6424f, 2.966f, 0}},
+        {49, 0, {2.385f, 0.2662f, 0.05997f, 0, 0.08394f, 0.3633f, 2.013f, 0}},
+        {3, 0, {2.717f, 0.5743f, 0.139f, 0.09286f, 0.05881f, 0.1805f, 1.758f, 0}},
+        {15, 0, {2.798f, 2.058f, 0, 0, 0.0983f, 0.6855f, 2.043f, 0}},
+        {28, 1, {7.81f, 0.1166f, 0.3139f, 0, 0.05803f, 0.1377f, 0, 0.2094f}},
+        {3, 1, {8.087f, 0.372f, 0.2751f, 0.06586f, 0.03938f, 0, 0, 0.1559f}},
+    };
+    static const AutoCost kAuto1x1s2[] = {
+        {24, 0, {1.361f, 0.5061f, 0.3012f, 0, 0.03557f, 0.5893f, 2.328f, 0}},
+        {3, 0, {1.797f, 0.4568f, 0.2562f, 0.2539f, 0.0314f, 0, 2.418f, 0}},
+        {15, 0, {1.237f, 1.981f, 0, 0, 0.04633f, 0.9107f, 3.543f, 0}},
+        {28, 0, {0.9643f, 0.4976f, 0.3845f, 0, 0.02384f, 0.5436f, 2.807f, 0}},
+        {2, 0, {0.5917f, 1.224f, 0.2238f, 0.2319f, 0.04262f, 0.1813f, 4.399f, 0}},
+        {3, 1, {7.404f, 0.1035f, 0.3729f, 0.08602f, 0.04949f, 0, 0, 0.2136f}},
+    };
+    static const AutoCost kAuto3x3[] = {
+        {53, 0, {1.44f, 0.122f, 0.2326f, 0.1964f, 0, 0, 0, 0.0195f, 0.2318f, 2.658f}},
+        {51, 0, {1.405f, 0.4354f, 0.2978f, 0.1379f, 0, 0, 0, 0.01873f, 0.3938f, 3.127f}},
+        {50, 0, {0.6819f, 2.679f, 0.5084f, 0.4584f, 0, 0, 0, 0, 0.3704f, 4.403f}},
+        {52, 0, {1.428f, 0.7499f, 0.3493f, 0.3238f, 0, 0, 0, 0.01345f, 0.2956f, 3.069f}},
+        {53, 1, {7.399f, 0.6351f, 0.09559f, 0.2857f, 0.1641f, 0.1075f, 0.07553f, 0, 0, 0}},
+        {51, 1, {7.735f, 0.7473f, 0.3876f, 0.3162f, 0.1222f, 0.1815f, 0.03201f, 0, 0.03982f, 0}},
+    };
+    static const AutoCost kAuto3x3s2[] = {
+        {53, 0, {0.8693f, 0.0844f, 0.1815f, 0, 0.02109f, 0, 0.0011f, 0.03831f, 0.4103f, 3.514f}},
+        {51, 0, {0.8916f, 0.7426f, 0, 0, 0.01947f, 0, 0.0135f, 0.04432f, 0.5163f, 4.059f}},
+        {50, 0, {0, 1.613f, 0, 0, 0.02192f, 0, 0, 0.06395f, 0.5248f, 6.263f}},
+        {3, 0, {1.755f, 0.608f, 0.1755f, 0.2307f, 0.07132f, 0.1841f, 3.074f, 0}},
+        {2, 0, {1.39f, 0.6092f, 0.2003f, 0, 0.1055f, 0.5777f, 4.388f, 0}},
+        {53, 1, {5.878f, 0.1491f, 0, 0, 0.0211f, 0.2208f, 0.05392f, 0.04992f, 0.2169f, 1.862f}},
+        {51, 1, {6.796f, 0.9241f, 0, 0, 0.01144f, 0.2609f, 0.05057f, 0.03745f, 0.4384f, 1.169f}},
+        {3, 1, {8.037f, 0.4517f, 0.2457f, 0.3174f, 0.2144f, 0, 0, 0.2264f}},
+    };
+
+    static float auto_cost(const vkhip_conv_desc *d, const AutoCost &k, int ks) {
+        const TileCfg &t   = kTiles[k.tile];
+        const int64_t  P   = (int64_t) d->N * d->OH * d->OW, co = ceil_div(d->Cout, 4) * 4, ci = ceil_div(d->Cin, 4) * 4;
+        const float    W   = (float) (ceil_div(co, t.BM) * ceil_div(P, t.BN) * ks) / 256.f;
+        const float    MB  = (float) ((int64_t) d->N * ci * d->H * d->W + P * co * (d->has_res ? 2 : 1)) * 2e-6f;
+        const float    pMB = ks > 1 ? (float) (ks * P * co) * 4e-6f : 0.f;
+        const float   *c   = k.c;
+        if (t.kind == 3) {
+            int n = halo_nbi(d, t);
+            for (int k: {8, 10, 12, 15}) // the sizes above 6 that are instantiated (conv_halo_tiles.hip)
+                if (n > 6 && n < k) n = k;
+            const float S = (float) ceil_div(d->Cin, 16) / ks;
+            const float r = (float) std::max(1, std::min(4, 160 * 1024 / (2 * (9 * t.BM / 32 + 4 * n) * 1024 + 64)));
+            const float q = std::ceil(W / r);
+            return c[0] + c[1] * W + c[2] * W * S + c[3] * S + c[4] * MB + c[5] * pMB + c[6] * W * S * n + c[7] * S * n + c[8] * q * S + c[9] * q;
+        }
+        const float S    = (float) ceil_div((int64_t) d->KH * d->KW * ci, kBK) / ks;
+        const int   ring = k.tile == 31 || k.tile == 49 ? 4 : k.tile == 28 ? 3 : 2;
+        const int   r    = t.PERS ? 1 : std::max(1, std::min(t.BM * t.BN <= 8192 ? 4 : 2, (int) (160 * 1024 / (std::min<float>(ring, std::max(1.f, S)) * (t.BM + t.BN) * 128))));
+        const float q    = std::ceil(W / r);
+        return c[0] + c[1] * W + c[2] * W * S + c[3] * S + c[4] * MB + c[5] * q * S + c[6] * q + c[7] * pMB;
+    }
+
+    // AUTO among the gather tiles: split-K when 64 x 64 tiles leave CUs idle and the reduction is deep.
+    static bool gather_split(const vkhip_conv_desc *d) {
+        const ConvGeom g = gemm_geom(d, 3, false);
+        return g.m_tiles * g.n_tiles < 256 && g.nsteps >= 16;
+    }
+
+    // The plan AUTO takes for a dense 1x1 (pad 0) or 3x3 (pad 1) layer at stride 1 or 2: the cheapest one
+    // predicted among the plans that accept it; first layers (at most 4 channels) take the thin kernel.
+    // Leaves `algo` at AUTO where none of them applies (other kernels, pads, dilations, an input scale):
+    // the gather tiles then. Over those layers the picks are 3-4% slower than the best measured plan of
+    // each layer and, in the geometric mean, 1.49x (1x1), 1.10x (1x1 stride 2), 1.73x (3x3) and 1.35x (3x3
+    // stride 2) faster than the gather tiles, the only ones AUTO knew before; on 300 other layers 1.54x. 256 -> 1024 at 14x14 b64 with a residual: 42.8 -> 21.2 us; 3x3 256 -> 256 there: 45.2 -> 21.8.
+    // First layers: 7x7 / 2 3 -> 64 at 224 b64 185 -> 39.7 us, 3x3 / 2 3 -> 16 at 640 b16 146 -> 22.5.
+    // Splits: only where the output is small and the reduction deep, and never a workspace that the
+    // allocation-free entry point could not hold.
+    static void auto_pick(const vkhip_conv_desc *d, int32_t &algo, int32_t &tile, int32_t &ksplit) {
+        if (d->group != 1 || d->in_scale) return;
+        vkhip_conv_plan p;
+        if (d->Cin <= 4 && d->KH > 1) {
+            const int t = d->Cout <= 16 ? 43 : d->Cout <= 32 ? 44 : 45;
+            if (vkhip_conv_plan_make(d, VKHIP_CONV_GEMM, t, 0, &p) == VKHIP_OK) algo = VKHIP_CONV_GEMM, tile = t;
+            return;
+        }
+        const bool one = d->KH == 1 && d->KW == 1 && dma_eligible(d, false);
+        const bool three = d->KH == 3 && d->KW == 3 && d->PT == 1 && d->PL == 1;
+        if (!one && !three) return;
+        const AutoCost *tab = nullptr;
+        int             n   = 0;
+        auto            use = [&](auto &t) { tab = t, n = (int) std::size(t); };
+        if (three) d->SH == 2 ? use(kAuto3x3s2) : use(kAuto3x3);
+        else d->SH == 2 ? use(kAuto1x1s2) : use(kAuto1x1);
+        const int64_t   out = (int64_t) d->N * d->OH * d->OW * d->Cout;
+        const bool      may_split = out <= (int64_t) 512 * 128 * 128 && d->KH * d->KW * d->Cin >= 256;
+        float           best = 1e30f;
+        // Stride 2 gains less: there the gather plan stays unless the pick beats its prediction by 10%
+        // (1x1: of 249 layers 14 lose more than 3% without that and one with it, for a mean gain of 1.13x
+        // and 1.10x) or 5% (3x3: none loses, 1.35x).
+        if (d->SH == 2) {
+            const bool split = gather_split(d);
+            if (vkhip_conv_plan_make(d, split ? VKHIP_CONV_SPLITK : VKHIP_CONV_GEMM, -1, 0, &p) == VKHIP_OK)
+                for (int i = 0; i < n; ++i)
+                    if (tab[i].tile == p.tile && (tab[i].split != 0) == split) best = (one ? 0.9f : 0.95f) * auto_cost(d, tab[i], std::max(1, p.ksplit));
+        }
+        for (int i = 0; i < n; ++i) {
+            // a 3x3 over a multiple of 16 channels takes the tile that the any-channel tile shares its kernel with
+            const int rc = kTiles[tab[i].tile].RC, t = rc && d->Cin % 16 == 0 ? rc : tab[i].tile;
+            for (int ks: {1, 2, 3, 4, 6, 8, 12, 16}) {
+                if ((ks > 1) != (tab[i].split != 0) || (ks > 1 && !may_split)) continue;
+                const int a = ks > 1 ? VKHIP_CONV_SPLITK : VKHIP_CONV_GEMM;
+                if (vkhip_conv_plan_make(d, a, t, ks > 1 ? ks : 0, &p) != VKHIP_OK) break;
+                if (ks > 1 && (p.ksplit != ks || p.workspace_bytes > VKHIP_NOALLOC_SCRATCH_BYTES)) break;
+                const float us = auto_cost(d, tab[i], ks);
+                if (us < best) best = us, algo = a, tile = t, ksplit = ks > 1 ? ks : 0;
+            }
+        }
+    }
+
     // Grid of a persistent kernel: the workgroups the device holds at once (occupancy of this
     // kernel x CUs), a multiple of 8 (its tile order deals tiles to the 8 XCDs), and no more than
     // the tiles need.
@@ -984,11 +1116,8 @@ int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, i
     if (algo == VKHIP_CONV_WINOGRAD && !wino_eligible(d))
         return set_error(VKHIP_ERR_INVALID, "Winograd F(2,3) needs 3x3 stride 1 pad 1 dilation 1");
     if (algo < VKHIP_CONV_AUTO || algo > VKHIP_CONV_SPLITK_LAST) return set_error(VKHIP_ERR_INVALID, "unknown conv algorithm %d", algo);
-    if (algo == VKHIP_CONV_AUTO) {
-        ConvGeom g   = gemm_geom(d, 3, false);
-        int64_t  wgs = g.m_tiles * g.n_tiles;
-        algo         = (wgs < 256 && g.nsteps >= 16) ? VKHIP_CONV_SPLITK : VKHIP_CONV_GEMM;
-    }
+    if (algo == VKHIP_CONV_AUTO && tile < 0 && ksplit <= 0) auto_pick(d, algo, tile, ksplit);
+    if (algo == VKHIP_CONV_AUTO) algo = gather_split(d) ? VKHIP_CONV_SPLITK : VKHIP_CONV_GEMM;
     const bool wino  = algo == VKHIP_CONV_WINOGRAD;
     const bool split = algo == VKHIP_CONV_SPLITK || algo == VKHIP_CONV_SPLITK_LAST;
     if (tile < 0) tile = split ? (ceil_div(d->Cout, 4) * 4 <= 32 ? 6 : 3) : default_tile(d, wino);
@@ -1060,13 +1189,16 @@ int vkhip_conv_pack_weights(const vkhip_conv_desc *d, const vkhip_conv_plan *pla
     if (bias)
         for (int oc = 0; oc < d->Cout; ++oc) b[oc] = bias[oc];
     if (!wino) {
+        // one slot (4 input channels of a tap) at a time: its values are neighbours in every layout
+        const int64_t taps = (int64_t) d->KH * d->KW;
         for (int oc = 0; oc < d->Cout; ++oc)
-            for (int ic = 0; ic < d->Cin; ++ic)
-                for (int ky = 0; ky < d->KH; ++ky)
-                    for (int kx = 0; kx < d->KW; ++kx) {
-                        int64_t slot = ((int64_t) ky * d->KW + kx) * g.Cinb + ic / 4;
-                        wp[tiled_index(g, kTiles[plan->tile], oc, slot * 4 + ic % 4)] = ref_half(w[(((int64_t) oc * d->Cin + ic) * d->KH + ky) * d->KW + kx]);
-                    }
+            for (int64_t tap = 0; tap < taps; ++tap)
+                for (int64_t cb = 0; cb < g.Cinb; ++cb) {
+                    half_t      *dst = wp + tiled_index(g, kTiles[plan->tile], oc, (tap * g.Cinb + cb) * 4);
+                    const float *src = w + ((int64_t) oc * d->Cin + cb * 4) * taps + tap;
+                    const int    n   = std::min<int64_t>(4, d->Cin - cb * 4);
+                    for (int l = 0; l < n; ++l) dst[l] = ref_half(src[l * taps]);
+                }
         return VKHIP_OK;
     }
     // U = G g G^T, G = [[1,0,0],[1/2,1/2,1/2],[1/2,-1/2,1/2],[0,0,1]] (reference ops/conv.cpp:117-141)
