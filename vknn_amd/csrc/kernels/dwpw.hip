@@ -6,28 +6,12 @@
 //   phase 2  the 1x1 projection as MFMA 32x32x16 GEMMs (A = packed pw weights streamed from L2,
 //            B = the LDS tile), then bias (+ residual) + activation and the fp16 NC4HW4 store.
 // Also hosts the fully-connected helper (a 1x1 conv over [N,K,1,1]).
-#include "common.h"
+#include "dwpw.h"
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
 namespace vkhip {
-
-    struct DwPwArgs {
-        const uint2  *x;
-        const float  *dw_b;  // [Eb*4]
-        const float  *dw_w;  // [Eb][KH][KW][4]
-        const float  *pw_b;  // [Coutp]
-        const half_t *pw_w;  // [Coutp][Kp]
-        const uint2  *res;
-        uint2        *y;
-        int           N, E, Eb, Ebp, H, W, OH, OW, KH, KW, SH, SW, PT, PL, DH, DW;
-        int           dw_act;
-        int           Cout, Coutb, m_frags, Kp, P;
-        int           act;
-        float         lo, hi;
-        int           has_res;
-    };
 
     template <int BN>
     __global__ __launch_bounds__(256) void dwpw_kernel(DwPwArgs a) {
@@ -972,6 +956,7 @@ int vkhip_dwpw_forward(const vkhip_dwpw_desc *d, const void *x, const void *blob
     a.Cout = d->Cout; a.Coutb = (int) g.Coutb; a.m_frags = (int) g.m_frags; a.Kp = (int) g.Kp;
     a.P = c.N * c.OH * c.OW;
     a.act = d->act; a.lo = d->act_lo; a.hi = d->act_hi; a.has_res = d->has_res;
+    a.dw_h = (const half_t *) (base + g.off_dwh);
     DwStrip t;
     int     RT = 0;
     // VKHIP_DWPW_STRIP=0 keeps the untiled kernel (A/B measurements)
@@ -985,6 +970,12 @@ int vkhip_dwpw_forward(const vkhip_dwpw_desc *d, const void *x, const void *blob
     DwRing rt;
     int    RTT = 0;
     if (ring_on && dwpw_ring_fits(d, g, kRingNS, rt, RTT)) {
+        // The column kernel reads the ring kernel's fp16 taps and was faster on all 32 shapes measured (its
+        // comment lists some), so the ring is left the 5x5 stride 1 convs with an odd left pad, whose
+        // windows do not fit. VKHIP_DWPW_COLS=0 keeps the ring kernel (A/B measurements).
+        const char *cols_env = std::getenv("VKHIP_DWPW_COLS");
+        DwPwCols    ct;
+        if (!(cols_env && cols_env[0] == '0') && dwpw_cols_plan(d, ct)) return dwpw_cols_launch(a, ct, resolve_stream(s));
         rt.x_bytes    = (int) (c.N * g.Eb * c.H * c.W * 8);
         rt.blob_bytes = (int) g.bytes;
         rt.off_dwb    = (int) g.off_dwb;
