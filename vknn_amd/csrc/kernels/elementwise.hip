@@ -265,35 +265,80 @@ namespace vkhip {
         }
     }
 
-    // y[n,c,p] = x[n,c,p] * s[n,c]; thread = two adjacent pixels of one 4-channel block.
-    __global__ void channel_scale_kernel(const uint2 *x, const uint2 *s, uint2 *y, int64_t Cb, int64_t HW, int64_t total) {
-        int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-        if (i >= total) return;
-        int64_t nc = i / HW; // n*Cb + cb
-        float4v sc = h4_to_f4(u2_as_h4(s[nc]));
-        float4v v  = h4_to_f4(u2_as_h4(x[i]));
-        y[i]       = h4_as_u2(f4_to_h4(v * sc));
+    // 16 bytes at an address that is a multiple of 8 (two pixels of a plane that may start at an odd one)
+    struct __attribute__((aligned(8))) px2 {
+        uint2 a, b;
+    };
+
+    // y[n,c,p] = x[n,c,p] * s[n,c]; thread = U pairs of adjacent pixels of the flattened planes, a block's
+    // width apart; where HW is odd (ODD) a pair can lie in two planes and the last one be half a pair.
+    // The fp16 product is the fp32 one rounded. I: unsigned, or int64_t past 2^31 pixels.
+    // Bound by memory; one pixel per thread (8 bytes, a 64-bit division) kept too little in flight:
+    // 128 x 672 x 14 x 14 (67 MB both ways) 13.8 -> 10.7 us, 32 x 96 x 112 x 112 34.9 -> 28.0 us, odd
+    // planes 64 x 64 x 55 x 55 10.4 -> 8.6 us.
+    template <typename I, bool ODD, int U = ODD ? 1 : 2>
+    __global__ void channel_scale_kernel(const uint2 *x, const uint2 *s, uint2 *y, I HW, I total) {
+        const I i0 = ((I) blockIdx.x * (blockDim.x * U) + threadIdx.x) * 2;
+        px2     v[U];
+        if (ODD && i0 + 1 == total) {
+            y[i0] = h4_as_u2(u2_as_h4(x[i0]) * u2_as_h4(s[i0 / HW]));
+            return;
+        }
+        if (i0 >= total) return;
+        half4 sa[U], sb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const I i = u && i0 + u * 512 >= total ? i0 : i0 + u * 512, nc = i / HW; // n*Cb + cb
+            v[u]      = *reinterpret_cast<const px2 *>(x + i);
+            sa[u]     = u2_as_h4(s[nc]);
+            sb[u]     = ODD ? u2_as_h4(s[i + 1 - nc * HW == HW ? nc + 1 : nc]) : sa[u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u && i0 + u * 512 >= total) return;
+            v[u].a = h4_as_u2(u2_as_h4(v[u].a) * sa[u]);
+            v[u].b = h4_as_u2(u2_as_h4(v[u].b) * sb[u]);
+            *reinterpret_cast<px2 *>(y + i0 + u * 512) = v[u];
+        }
     }
 
-    // L lanes per (n, cb) plane (L a power of two from 8 to 64, about one lane per 8 pixels): mean
-    // over HW pixels of 4 channels (fp32 sums), lane partials reduced with shuffles. Small planes
-    // (7x7 before a classifier) would leave most of a full wave idle.
-    __global__ void gap_kernel(const uint2 *x, uint2 *y, int64_t NCb, int64_t HW, int L) {
+    // L lanes per (n, cb) plane (L a power of two from 8 to 64, about one lane per 8 pixels): mean over
+    // HW pixels of 4 channels (fp32 sums). Small planes (7x7 before a classifier) would leave most of a
+    // full wave idle. A lane has four loads of two pixels in flight. The lanes' partials are reduced so
+    // that lane l ends with channel l % 4: two exchanges, then one, then one per further halving.
+    // Bound by memory, on large planes by the loads a lane has in flight. One pixel per load, one load in
+    // flight, four values exchanged per halving -> now: 128 x 672 x 14 x 14 (34 MB) 9.8 -> 6.8 us,
+    // 128 x 72 x 28 x 28 7.0 -> 4.5 us, 32 x 96 x 112 x 112 61.9 -> 14.6 us, 128 x 960 x 7 x 7 4.6 -> 3.9 us.
+    template <typename I>
+    __global__ void gap_kernel(const uint2 *x, half_t *y, int64_t NCb, I HW, int lg) {
         const int64_t t    = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-        const int64_t w    = t / L;
-        const int     lane = (int) (t % L);
+        const int     L    = 1 << lg;
+        const int64_t w    = t >> lg;
+        const int     lane = (int) t & (L - 1);
         float4v       s    = {0.f, 0.f, 0.f, 0.f};
         if (w < NCb) {
             const uint2 *src = x + w * HW;
-            for (int64_t p = lane; p < HW; p += L) s += h4_to_f4(u2_as_h4(src[p]));
+            const I      P   = HW >> 1; // pixel pairs
+            for (I p0 = lane; p0 < P; p0 += 4 * L) {
+                px2 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const px2 *>(src + 2 * (p0 + u * L < P ? p0 + u * L : p0));
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const unsigned in = p0 + u * L < P ? ~0u : 0u; // a mask, as a branch would part the loads
+                    s += h4_to_f4(u2_as_h4(uint2 {v[u].a.x & in, v[u].a.y & in})) + h4_to_f4(u2_as_h4(uint2 {v[u].b.x & in, v[u].b.y & in}));
+                }
+            }
+            if ((HW & 1) && lane == 0) s += h4_to_f4(u2_as_h4(src[HW - 1]));
         }
-        for (int off = L >> 1; off > 0; off >>= 1) {
-            s.x += __shfl_xor(s.x, off);
-            s.y += __shfl_xor(s.y, off);
-            s.z += __shfl_xor(s.z, off);
-            s.w += __shfl_xor(s.w, off);
-        }
-        if (w < NCb && lane == 0) y[w] = h4_as_u2(f4_to_h4(s / (float) HW));
+        const bool o1 = lane & 1, o2 = lane & 2;
+        float      k0 = o1 ? s.y : s.x, k1 = o1 ? s.w : s.z; // channels lane % 2 and lane % 2 + 2
+        k0 += __shfl_xor(o1 ? s.x : s.y, 1);
+        k1 += __shfl_xor(o1 ? s.z : s.w, 1);
+        float m = o2 ? k1 : k0;
+        m += __shfl_xor(o2 ? k0 : k1, 2);
+        for (int off = 4; off < L; off <<= 1) m += __shfl_xor(m, off);
+        if (w < NCb && lane < 4) y[w * 4 + lane] = (half_t) (m / (float) HW);
     }
 
     // Max pool over NC4HW4; out-of-image taps are skipped (reference maxpool.cpp semantics).
@@ -690,16 +735,26 @@ int vkhip_binary(const void *a, const void *b, void *y, int64_t n, int32_t op, v
 int vkhip_channel_scale(const void *x, const void *scale, void *y, int64_t N, int64_t C, int64_t HW, vkhip_stream_t s) {
     if (!x || !scale || !y || N <= 0 || C <= 0 || HW <= 0) return set_error(VKHIP_ERR_INVALID, "channel_scale: bad arguments");
     int64_t Cb = ceil_div(C, 4), total = N * Cb * HW;
-    channel_scale_kernel<<<grid1(total), 256, 0, resolve_stream(s)>>>((const uint2 *) x, (const uint2 *) scale, (uint2 *) y, Cb, HW, total);
+    auto go = [&](auto kernel, auto i, int per_thread) {
+        typedef decltype(i) I;
+        kernel<<<grid1(ceil_div(total, per_thread)), 256, 0, resolve_stream(s)>>>((const uint2 *) x, (const uint2 *) scale, (uint2 *) y, (I) HW, (I) total);
+    };
+    const bool odd = HW % 2, small = total < (1LL << 31);
+    if (small && !odd) go(channel_scale_kernel<unsigned, false>, 0u, 4);
+    else if (small) go(channel_scale_kernel<unsigned, true>, 0u, 2);
+    else if (!odd) go(channel_scale_kernel<int64_t, false>, int64_t {}, 4);
+    else go(channel_scale_kernel<int64_t, true>, int64_t {}, 2);
     return check_launch("channel_scale");
 }
 
 int vkhip_global_avg_pool(const void *x, void *y, int64_t N, int64_t C, int64_t H, int64_t W, vkhip_stream_t s) {
     if (!x || !y || N <= 0 || C <= 0 || H <= 0 || W <= 0) return set_error(VKHIP_ERR_INVALID, "gap: bad arguments");
     int64_t NCb = N * ceil_div(C, 4);
-    int L = 8;
-    while (L < 64 && L * 8 < H * W) L <<= 1;
-    gap_kernel<<<grid1(NCb * L), 256, 0, resolve_stream(s)>>>((const uint2 *) x, (uint2 *) y, NCb, H * W, L);
+    int lg = 3;
+    while (lg < 6 && (8LL << lg) < H * W) ++lg;
+    const int64_t L = 1LL << lg;
+    if (H * W < (1LL << 30)) gap_kernel<int><<<grid1(NCb * L), 256, 0, resolve_stream(s)>>>((const uint2 *) x, (half_t *) y, NCb, (int) (H * W), lg);
+    else gap_kernel<int64_t><<<grid1(NCb * L), 256, 0, resolve_stream(s)>>>((const uint2 *) x, (half_t *) y, NCb, H * W, lg);
     return check_launch("global_avg_pool");
 }
 
