@@ -1,6 +1,8 @@
 """Network-level parity: the vknn Session on the HIP backend (through include/vknn_c.h) against the
 CPU oracle on the same seeded graphs and inputs. Bar: max|d|/max|ref| <= 2e-2, cosine >= 0.9999
 per output tensor. The input is fp32 NCHW on both sides (the HIP path packs it to fp16 itself)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -78,6 +80,16 @@ def test_config2_resnet50_b1(gpu):
     sess = V.Session("resnet50", 1, seed=7)
     x = make_input(sess.in_shape, 2)
     check_outputs(sess.run(x), oracle_model_run("resnet50", 1, 7, x), sess.out_elems, "resnet50 b1")
+
+
+def test_split_plans_stay_in_the_tuned_set(gpu):
+    """A split sums its fp32 partials in an order of its own, so the splits that a session chooses
+    among decide what its outputs round to: batch-1 ResNet-50 keeps to the set its layers were
+    compared on (hip_backend.cpp, choosePlan)."""
+    plan = V.Session("resnet50", 1, seed=7).describe()
+    splits = set(re.findall(r"splitk(?:_last)? tile=(\d+) ksplit=(\d+)", plan))
+    assert splits and {int(t) for t, _ in splits} <= {1, 3, 6, 8, 10, 14, 16, 17, 18, 20, 26}, splits
+    assert {int(k) for _, k in splits} <= {2, 3, 4, 8, 16}, splits
 
 
 def test_device_input_path_matches_host_path(gpu):

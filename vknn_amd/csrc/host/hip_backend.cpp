@@ -305,15 +305,21 @@ namespace vknn {
                     for (int rt: {0, 4, 7, 14, 204, 207, 404, 407, 907, 914})
                         if (rt < 100 || !(std::getenv("VKNN_HIP_DW_PIPE") && std::getenv("VKNN_HIP_DW_PIPE")[0] == '0'))
                             cands.push_back({VKHIP_CONV_DEPTHWISE, rt, 0});
+                // the heuristic pick among the gather tiles (AUTO with a given tile only chooses whether to
+                // split): the tiles that AUTO's cost model chooses from are candidates by themselves
                 vkhip_conv_plan base;
-                check(vkhip_conv_plan_make(&d, VKHIP_CONV_AUTO, -1, 0, &base), "conv plan");
+                int32_t         balgo = VKHIP_CONV_AUTO;
+                if (!dw && !d.in_scale) {
+                    check(vkhip_conv_plan_make(&d, VKHIP_CONV_AUTO, 3, 0, &base), "conv plan");
+                    balgo = base.algo;
+                }
+                check(vkhip_conv_plan_make(&d, balgo, -1, 0, &base), "conv plan");
                 int64_t pixels = (int64_t) d.N * d.OH * d.OW;
                 // Split-K when the direct grid cannot fill the device (fewer than ~2 workgroups per CU
                 // with the big tiles) and the reduction is deep enough to split.
                 const int64_t kdepth = (int64_t) d.KH * d.KW * ((d.Cin + 3) / 4) * 4;
                 if (!dw && (pixels <= 4096 || base.algo == VKHIP_CONV_SPLITK || (pixels * (int64_t) d.Cout <= (int64_t) 512 * 128 * 256 && kdepth >= 512))) {
-                    // (the any-channel halo tiles only where the tiles they share their kernels with refuse)
-                    for (int t: d.Cin % 16 ? std::vector<int> {3, 8, 10, 14, 24, 28, 51, 53} : std::vector<int> {3, 10, 14, 16, 20, 24, 26, 28, 33})
+                    for (int t: {3, 6, 1, 8, 10, 14, 16, 17, 18, 20, 26})
                         for (int ks: {2, 3, 4, 8, 16})
                             for (int alg: {VKHIP_CONV_SPLITK, VKHIP_CONV_SPLITK_LAST}) cands.push_back({alg, t, ks});
                 }
