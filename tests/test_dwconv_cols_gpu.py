@@ -51,6 +51,19 @@ def test_cols_pads(gpu, k, s, pads):
     assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
 
 
+@pytest.mark.parametrize("k,s,p", [(3, 1, 7), (3, 1, 8), (5, 1, 10), (3, 2, 10), (5, 2, 12)])
+def test_cols_bands_in_the_top_padding(gpu, k, s, p):
+    """A plane split into 4-row bands whose first band lies wholly above the image: its outputs see
+    padding only, in every plane (a row of the plane before is no row of this one)."""
+    x, w, b, d, ys, _ = case((1, 16, 20, 20), k, s, (p,) * 4, 0, False)
+    got, plan, _ = gpu_conv(x, w, b, (s, s), (p,) * 4, group=16)
+    assert plan.tile == 0
+    ref = oracle_conv(x, w, b, (s, s), (p,) * 4, group=16)
+    assert np.array_equal(got[:, :, :1], np.broadcast_to(b.astype(np.float16).astype(np.float32)[None, :, None, None], got[:, :, :1].shape))
+    rel, cos = parity(got, ref)
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
 @pytest.mark.parametrize("k,s", [(3, 1), (3, 2), (5, 1), (5, 2)])
 def test_cols_infinities_stay_in_their_window(gpu, k, s):
     p = k // 2

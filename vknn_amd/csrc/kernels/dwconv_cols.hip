@@ -90,7 +90,7 @@ namespace vkhip {
             __builtin_amdgcn_make_buffer_rsrc((void *) (a.has_res ? a.res : a.y), (short) 0, a.has_res ? a.N * a.Cb * OH * OW * 8 : 0, 0x00020000);
         // rows of the band inside the image; the others read zeros
         const int R    = t.BR * S + K - S; // input rows of a band
-        const int ylast = min(H, iy0 + R);
+        const int ylast = max(0, min(H, iy0 + R)); // 0: the whole band lies in the top padding
         auto load = [&](int r) __attribute__((always_inline)) {
             const bool     row = (unsigned) (iy0 + r) < (unsigned) ylast;
             const unsigned o   = xb + (unsigned) (r * W8);
