@@ -78,6 +78,28 @@ def test_cols_infinities_stay_in_their_window(gpu, k, s):
     assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
 
 
+@pytest.mark.parametrize("k,s", [(3, 1), (3, 2), (5, 1), (5, 2)])
+@pytest.mark.parametrize("pooled", [False, True])
+def test_cols_residual_in_place_beside_infinities(gpu, k, s, pooled):
+    """A residual that is the output's own memory gives the bits of one that is not, also in windows
+    whose outputs are computed again tap by tap."""
+    lib, p = V.vkhip(), k // 2
+    x, w, b, d, ys, rr = case((2, 8, 17, 22), k, s, (p,) * 4, 0, True)
+    x[0, 2, 5, 7], x[1, 6, 0, 21], x[1, 1, 16, 0] = np.inf, -np.inf, np.nan
+    ref, plan, _ = gpu_conv(x, w, b, (s, s), (p,) * 4, group=8, res=rr)
+    assert not np.isfinite(ref).all()
+    blob = np.zeros(plan.weight_bytes, np.uint8)
+    check(lib.vkhip_conv_pack_weights(ctypes.byref(d), ctypes.byref(plan), w.ctypes.data, b.ctypes.data, blob.ctypes.data))
+    dx, db, dy = to_device_nc4(x), V.DeviceBuffer.from_array(blob), to_device_nc4(rr)
+    if pooled:
+        dp = V.DeviceBuffer(2 * 2 * lib.vkhip_conv_pool_parts(ctypes.byref(d), ctypes.byref(plan)) * 16)
+        check(lib.vkhip_conv_forward_pooled(ctypes.byref(d), ctypes.byref(plan), dx.ptr, db.ptr, dy.ptr, dy.ptr, dp.ptr, None))
+    else:
+        check(lib.vkhip_conv_forward(ctypes.byref(d), ctypes.byref(plan), dx.ptr, db.ptr, dy.ptr, dy.ptr, None, None))
+    check(lib.vkhip_stream_sync(None))
+    np.testing.assert_array_equal(from_device_nc4(dy, ys), ref)
+
+
 @pytest.mark.parametrize("shape,k,s", [((3, 22, 14, 14), 3, 1), ((4, 960, 7, 7), 5, 1), ((2, 12, 29, 31), 5, 2), ((1, 8, 40, 9), 3, 2)])
 def test_cols_pool_sums(gpu, shape, k, s):
     """The parts of a plane add up to the sum of the stored fp16 outputs: fp32 sums of at most

@@ -36,8 +36,9 @@ namespace vkhip {
     };
 
     // POOL: also leave the pool sums (without them the kernel holds fewer registers: 15.4 -> 15.0 us on the
-    // first shape above).
-    template <int K, int S, int ACT, bool ODD, bool POOL>
+    // first shape above). RES: with a residual (as a run-time branch of each row 15.3 us, as a variant
+    // 14.2; both without a residual).
+    template <int K, int S, int ACT, bool ODD, bool POOL, bool RES>
     __global__ __launch_bounds__(256, 4) void dwconv_cols_kernel(DwArgs a, DwCols t) {
         using Sh = DwColsShape<K, S>;
         constexpr int      F = Sh::F, U = Sh::U, DX = Sh::DX;
@@ -87,7 +88,7 @@ namespace vkhip {
         const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void *) a.x, (short) 0, a.N * a.Cb * H * W * 8, 0x00020000);
         const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc((void *) a.y, (short) 0, a.N * a.Cb * OH * OW * 8, 0x00020000);
         const __amdgpu_buffer_rsrc_t rrs =
-            __builtin_amdgcn_make_buffer_rsrc((void *) (a.has_res ? a.res : a.y), (short) 0, a.has_res ? a.N * a.Cb * OH * OW * 8 : 0, 0x00020000);
+            __builtin_amdgcn_make_buffer_rsrc((void *) (RES ? a.res : a.y), (short) 0, RES ? a.N * a.Cb * OH * OW * 8 : 0, 0x00020000);
         // rows of the band inside the image; the others read zeros
         const int R    = t.BR * S + K - S; // input rows of a band
         const int ylast = max(0, min(H, iy0 + R)); // 0: the whole band lies in the top padding
@@ -111,9 +112,17 @@ namespace vkhip {
         const unsigned yb   = (unsigned) ((plane * OH + y0) * OW + ox) * 8u;
         const bool     rag  = (a.C & 3) != 0;
         float4v        psum = {0.f, 0.f, 0.f, 0.f};
-        auto finish = [&](float4v v, int y, bool ok) __attribute__((always_inline)) {
+        float          nf   = 0.f; // NaN once a sum of this lane was not finite
+        int            kept = 0;   // RES: the rows stored until then
+        auto finish = [&](float4v v, int y, bool ok, auto first_c) __attribute__((always_inline)) {
+            // The residual may be the output's own memory: its rows from the first non-finite sum on are
+            // left as they are for the recomputation (without one they are stored twice).
+            if constexpr (RES && decltype(first_c)::value) {
+                ok = ok && nf == nf;
+                kept += nf == nf;
+            }
             const unsigned o = ok ? yb + (unsigned) (y * OW) * 8u : kInvalid;
-            if (a.has_res) v += h4_to_f4(__builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(rrs, o, 0, kStreamLoad)));
+            if constexpr (RES) v += h4_to_f4(__builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(rrs, o, 0, kStreamLoad)));
             v.x = apply_act(v.x, ACT, a.lo, a.hi);
             v.y = apply_act(v.y, ACT, a.lo, a.hi);
             v.z = apply_act(v.z, ACT, a.lo, a.hi);
@@ -137,10 +146,9 @@ namespace vkhip {
                 psum.w = __builtin_fmaf((float) hs.w, 1.f, psum.w);
             }
         };
-        float nf = 0.f; // NaN once a sum of this lane was not finite
         auto emit = [&](const float4v &v, int y) __attribute__((always_inline)) {
             nf = __builtin_fmaf(v.x, 0.f, nf);
-            finish(v, y + dyl, xok && y + dyl < ylim);
+            finish(v, y + dyl, xok && y + dyl < ylim, std::true_type {});
         };
 
         u32x4 buf[U];
@@ -192,9 +200,9 @@ namespace vkhip {
         }
         if (__any(nf != nf)) {
             if (nf != nf && xok) {
-                psum = float4v {0.f, 0.f, 0.f, 0.f};
+                if constexpr (!RES) psum = float4v {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-                for (int y = dyl; y < ylim; y += S) {
+                for (int y = dyl + kept * S; y < ylim; y += S) {
                     float4v v = b0;
 #pragma unroll 1
                     for (int k = 0; k < K * K; ++k) {
@@ -206,7 +214,7 @@ namespace vkhip {
                         v.z = __builtin_fmaf((float) xv.z, (float) wv.z, v.z);
                         v.w = __builtin_fmaf((float) xv.w, (float) wv.w, v.w);
                     }
-                    finish(v, y, true);
+                    finish(v, y, true, std::false_type {});
                 }
             }
         }
@@ -266,8 +274,15 @@ namespace vkhip {
         const dim3 grid((unsigned) ceil_div((int64_t) t.groups * a.Cb, 4));
         auto       go = [&](auto act_c) {
             constexpr int ACT = decltype(act_c)::value;
-            if (a.W % 2) a.pool ? dwconv_cols_kernel<K, S, ACT, true, true><<<grid, 256, 0, st>>>(a, t) : dwconv_cols_kernel<K, S, ACT, true, false><<<grid, 256, 0, st>>>(a, t);
-            else a.pool ? dwconv_cols_kernel<K, S, ACT, false, true><<<grid, 256, 0, st>>>(a, t) : dwconv_cols_kernel<K, S, ACT, false, false><<<grid, 256, 0, st>>>(a, t);
+            auto          with = [&](auto odd_c, auto pool_c) {
+                constexpr bool ODD = decltype(odd_c)::value, POOL = decltype(pool_c)::value;
+                if (a.has_res) dwconv_cols_kernel<K, S, ACT, ODD, POOL, true><<<grid, 256, 0, st>>>(a, t);
+                else dwconv_cols_kernel<K, S, ACT, ODD, POOL, false><<<grid, 256, 0, st>>>(a, t);
+            };
+            using std::false_type;
+            using std::true_type;
+            if (a.W % 2) a.pool ? with(true_type {}, true_type {}) : with(true_type {}, false_type {});
+            else a.pool ? with(false_type {}, true_type {}) : with(false_type {}, false_type {});
         };
         using std::integral_constant;
         switch (a.act) {
