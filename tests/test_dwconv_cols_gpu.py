@@ -41,6 +41,23 @@ def test_cols_against_oracle(gpu, shape, act, res, k, s):
     assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
 
 
+@pytest.mark.parametrize("shape,k,s,tile", [((2, 6, 9, 14), 3, 1, 0), ((1, 8, 6, 300), 5, 1, 0), ((2, 5, 15, 33), 5, 2, 0), ((2, 6, 9, 14), 3, 1, 4),
+                                            ((2, 8, 28, 28), 5, 1, 207), ((9, 12, 7, 7), 3, 1, 907), ((1, 8, 6, 300), 7, 1, 0)])
+@pytest.mark.parametrize("res", [False, True])
+def test_hard_sigmoid(gpu, shape, k, s, tile, res):
+    """clamp(lo v + hi, 0, 1) on every depthwise kernel (columns, also on rows wider than a strip;
+    strips, pipelined and persistent ones; any shape): the oracle's plain sums, then the formula,
+    which the kernel applies to its own fp32 sums before the rounding to fp16."""
+    p = k // 2
+    x, w, b, d, ys, rr = case(shape, k, s, (p,) * 4, 6, res)
+    lo, hi = 0.2, 0.5
+    got, plan, _ = gpu_conv(x, w, b, (s, s), (p,) * 4, group=shape[1], act=6, lo=lo, hi=hi, res=rr, algo=V.CONV_DEPTHWISE, tile=tile)
+    ref = np.clip(lo * oracle_conv(x, w, b, (s, s), (p,) * 4, group=shape[1], res=rr) + hi, 0, 1)
+    assert ref.min() == 0 and ref.max() == 1
+    rel, cos = parity(got, ref)
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
 # pads (top, left, bottom, right); 5x5 stride 1 with an odd left pad does not fit the window: strip kernel
 @pytest.mark.parametrize("k,s,pads", [(3, 1, (0, 0, 0, 0)), (3, 2, (0, 0, 1, 1)), (3, 1, (2, 2, 2, 2)), (5, 2, (1, 1, 2, 2)), (5, 1, (1, 1, 1, 1)),
                                       (5, 1, (0, 0, 4, 4)), (5, 1, (4, 4, 0, 0)), (3, 2, (3, 3, 3, 3))])

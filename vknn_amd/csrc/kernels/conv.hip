@@ -480,6 +480,7 @@ namespace vkhip {
             case VKHIP_ACT_CLIP: finish(std::integral_constant<int, VKHIP_ACT_CLIP> {}); break;
             case VKHIP_ACT_HARDSWISH: finish(std::integral_constant<int, VKHIP_ACT_HARDSWISH> {}); break;
             case VKHIP_ACT_SILU: finish(std::integral_constant<int, VKHIP_ACT_SILU> {}); break;
+            case VKHIP_ACT_HARDSIGMOID: finish(std::integral_constant<int, VKHIP_ACT_HARDSIGMOID> {}); break;
             default: finish(std::integral_constant<int, VKHIP_ACT_NONE> {}); break;
         }
         if (a.pool) {

@@ -291,6 +291,7 @@ namespace vkhip {
             case VKHIP_ACT_CLIP: go(integral_constant<int, VKHIP_ACT_CLIP> {}); break;
             case VKHIP_ACT_HARDSWISH: go(integral_constant<int, VKHIP_ACT_HARDSWISH> {}); break;
             case VKHIP_ACT_SILU: go(integral_constant<int, VKHIP_ACT_SILU> {}); break;
+            case VKHIP_ACT_HARDSIGMOID: go(integral_constant<int, VKHIP_ACT_HARDSIGMOID> {}); break;
             default: go(integral_constant<int, VKHIP_ACT_NONE> {}); break;
         }
     }
