@@ -171,7 +171,8 @@ typedef struct vkhip_conv_plan {
     int32_t algo;            /* one of VKHIP_CONV_* (never AUTO once planned) */
     int32_t tile;            /* GEMM tile configuration index (see vkhip_conv_tile_count) */
     int32_t ksplit;          /* split-K parts (SPLITK only) */
-    int32_t reserved;
+    int32_t reserved;        /* for reports, not read by forward calls: 3x3 halo tiles, the 1 KB copies
+                              * per channel slot of the largest input band (0 for other tiles) */
     size_t  weight_bytes;    /* size of the packed weight blob */
     size_t  workspace_bytes; /* device scratch the forward call needs (0 = none) */
 } vkhip_conv_plan;

@@ -4,6 +4,7 @@ allocation-free entry point holds, and shapes that none of the modelled kernels 
 plan. The picks' results are compared with the oracle in test_conv_sweep_gpu.py."""
 import ctypes
 import random
+import time
 
 import pytest
 
@@ -45,3 +46,53 @@ def test_auto_with_a_given_tile_or_split_keeps_it():
     for t in (0, 3, 24):
         rc, p = plan_of(V.CONV_AUTO, t, 0, **c)
         assert rc == 0 and p.tile == t
+
+
+def band_copies(d, bn, slots, waves):
+    """The 1 KB copies per channel slot of a halo tile's largest band, by walking every tile."""
+    ohw, p, rows = d.OH * d.OW, d.N * d.OH * d.OW, 0
+    for p0 in range(0, p, bn):
+        p1 = min(p, p0 + bn) - 1
+        rows = max(rows, (p1 // ohw - p0 // ohw) * (d.H + 2) + d.SH * (p1 % ohw // d.OW - p0 % ohw // d.OW) + 3)
+    n = -(-rows * (((d.W + 3) & ~1) // 2) // 64)
+    while slots * n % waves:
+        n += 1
+    return n
+
+
+# tile -> (pixels, channel slots, waves of a workgroup); most copies its kernels are built for
+HALO = {18: (256, 4, 4, 15), 26: (128, 4, 4, 8), 19: (256, 4, 4, 10), 50: (256, 4, 4, 15), 53: (128, 4, 4, 8)}
+
+
+def test_halo_band_matches_the_walk_over_all_tiles():
+    """A halo plan's band, found without walking the layer's tiles, over random layers: tiles that
+    divide an image or not, one image or many, rows shorter and longer than a tile."""
+    r, made = random.Random(5), 0
+    for _ in range(1500):
+        s, big = r.choice((1, 2)), r.random()
+        h, w = (r.randint(1, 90 if big < 0.2 else 24) for _ in range(2))
+        tile = r.choice(list(HALO))
+        bn, slots, waves, most = HALO[tile]
+        c = dict(N=r.randint(1, 40 if big < 0.2 else 140), Cin=32, H=h, W=w, Cout=32, OH=(h - 1) // s + 1, OW=(w - 1) // s + 1, KH=3, KW=3, SH=s, SW=s, PT=1, PL=1)
+        rc, p = plan_of(V.CONV_GEMM, tile, 0, **c)
+        want = band_copies(V.ConvDesc(**c), bn, slots, waves)
+        assert (rc == 0) == (want <= most), (tile, c, want)
+        if rc == 0:
+            made += 1
+            assert p.reserved == want, (tile, c, want)
+    assert made > 300
+
+
+def test_plans_of_large_maps_cost_no_walk():
+    """Host time of a plan does not grow with the number of tiles (12800 here, which took 29 us per call
+    to walk): best of several, against the same layer on one image."""
+    best = {}
+    for n in (1, 128):
+        c = dict(N=n, Cin=16, H=80, W=80, Cout=16, OH=80, OW=80, KH=3, KW=3, SH=1, SW=1, PT=1, PL=1)
+        best[n] = 1e9
+        for _ in range(30):
+            t = time.perf_counter()
+            for _ in range(20):
+                assert plan_of(V.CONV_GEMM, 33, 0, **c)[0] == 0
+            best[n] = min(best[n], (time.perf_counter() - t) / 20)
+    assert best[128] < best[1] + 10e-6, best

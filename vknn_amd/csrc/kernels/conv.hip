@@ -691,20 +691,61 @@ namespace vkhip {
                (t.RC || d->Cin % (16 * t.KK) == 0);
     }
 
-    // 1 KB copy chunks per channel slot of the largest input band any workgroup of a halo tile
-    // needs: band rows run from the row above the first output pixel's row to the row below the
-    // last one's, with two extra (zero) rows per image boundary crossed; W/2 + 1 pixel pairs a row.
-    static int halo_nbi(const vkhip_conv_desc *d, const TileCfg &t) {
-        const int64_t OHW = (int64_t) d->OH * d->OW, P = (int64_t) d->N * OHW, PW = ((d->W + 3) & ~1) / 2, S = d->SH;
+    // Smallest k >= 0 with lo <= k * a mod m <= hi (0 <= lo <= hi < m), or -1: Euclid's steps on (a, m).
+    static int64_t first_multiple_in(int64_t a, int64_t m, int64_t lo, int64_t hi) {
+        if (lo == 0) return 0;
+        a %= m;
+        if (a == 0) return -1;
+        if (2 * a > m) return first_multiple_in(m - a, m, m - hi, m - lo);
+        const int64_t k = ceil_div(lo, a);
+        if (k * a <= hi) return k;
+        // no multiple of a in the range itself: the fewest wraps y that bring one into [lo + y m, hi + y m]
+        const int64_t y = first_multiple_in(m % a, a, a - hi % a, a - lo % a);
+        return y < 0 ? -1 : ceil_div(lo + y * m, a);
+    }
+
+    // Band rows of the largest input band any workgroup of a halo tile needs: from the row above the
+    // first output pixel's row to the row below the last one's, with two extra (zero) rows per image
+    // boundary crossed. Tile k starts at pixel r = k * BN mod OHW of an image, and its rows depend on r
+    // only through how many output rows (d or d + 1 by the column) and image ends (two cases by the row)
+    // lie up to its last pixel: of these four cases the largest that some full tile meets, and the
+    // ragged last tile. Every forward call of a halo plan asks for it, so the tiles are not walked (29 us
+    // of host time at 16 -> 16 channels of 80x80, batch 128; 0.2 us now).
+    static int64_t halo_rows(const vkhip_conv_desc *d, const TileCfg &t) {
+        const int64_t OW = d->OW, OH = d->OH, OHW = OH * OW, P = (int64_t) d->N * OHW, S = d->SH, full = P / t.BN;
         int64_t       rows = 0;
-        for (int64_t p0 = 0; p0 < P; p0 += t.BN) {
-            const int64_t p1 = std::min(P, p0 + t.BN) - 1;
-            const int64_t nf = p0 / OHW, oyf = (p0 % OHW) / d->OW;
-            const int64_t nl = p1 / OHW, oyl = (p1 % OHW) / d->OW;
-            rows = std::max(rows, (nl - nf) * (d->H + 2) + S * (oyl - oyf) + 1 + 2);
+        if (P % t.BN) {
+            const int64_t p0 = full * t.BN, p1 = P - 1;
+            rows = (p1 / OHW - p0 / OHW) * (d->H + 2) + S * ((p1 % OHW) / OW - (p0 % OHW) / OW) + 3;
         }
-        int nbi = (int) ceil_div(rows * PW, 64);
-        const int nw = t.WM * t.WN;
+        const int64_t rem = (t.BN - 1) % OW;
+        for (int j = 1; j >= 0 && full; --j) {
+            const int64_t D = (t.BN - 1) / OW + j, x0 = j ? OW - rem : 0, x1 = j ? OW - 1 : OW - 1 - rem; // columns that give D
+            if (x0 > x1) continue;
+            for (int h = 1; h >= 0; --h) {
+                const int64_t n = D / OH + h; // image ends crossed, from output rows y0 .. y1
+                const int64_t y0 = std::max<int64_t>(0, n * OH - D), y1 = std::min<int64_t>(OH - 1, (n + 1) * OH - 1 - D);
+                const int64_t v = n * (d->H + 2) + S * (D - n * OH) + 3;
+                if (y0 > y1 || v <= rows) continue;
+                // a tile that starts in those columns at all (OW divides OHW), then in those rows
+                const int64_t k = first_multiple_in(t.BN, OW, x0, x1);
+                if (k < 0 || k >= full) continue;
+                bool hit = k * t.BN % OHW / OW >= y0 && k * t.BN % OHW / OW <= y1;
+                for (int64_t y = y1; y >= y0 && !hit; --y) {
+                    const int64_t q = first_multiple_in(t.BN, OHW, y * OW + x0, y * OW + x1);
+                    hit = q >= 0 && q < full;
+                }
+                if (hit) rows = v;
+            }
+        }
+        return rows;
+    }
+
+    // 1 KB copy chunks per channel slot of that band (W/2 + 1 pixel pairs a row), a multiple that every
+    // wave copies the same number of.
+    static int halo_nbi(const vkhip_conv_desc *d, const TileCfg &t) {
+        int       nbi = (int) ceil_div(halo_rows(d, t) * (((d->W + 3) & ~1) / 2), 64);
+        const int nw  = t.WM * t.WN;
         while ((4 * t.KK * nbi) % nw) ++nbi;
         return nbi;
     }
@@ -1128,7 +1169,8 @@ int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, i
     if (d->has_res == 2 && (wino || kTiles[tile].kind == 4))
         return set_error(VKHIP_ERR_UNSUPPORTED, "a residual after the activation runs on GEMM / split-K plans of the gather, B-direct, LDS-DMA, "
                          "halo and thin tiles only");
-    if (kTiles[tile].kind == 3 && (wino || !halo_shape_ok(d, kTiles[tile]) || halo_nbi(d, kTiles[tile]) > kHaloMaxNBI[tile]))
+    const int nbi = kTiles[tile].kind == 3 && !wino && halo_shape_ok(d, kTiles[tile]) ? halo_nbi(d, kTiles[tile]) : 0;
+    if (kTiles[tile].kind == 3 && (!nbi || nbi > kHaloMaxNBI[tile]))
         return set_error(VKHIP_ERR_UNSUPPORTED, "tile %d needs a 3x3 stride-1/2 pad-1 conv with Cin %% %d == 0 and a band that fits LDS", tile,
                          16 * kTiles[tile].KK);
     if (kTiles[tile].kind == 4 && (wino || !stem_shape_ok(d) || stem_nbi(d, kTiles[tile]) > kHaloMaxNBI[tile]))
@@ -1145,8 +1187,9 @@ int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, i
     if (kTiles[tile].PERS && (algo != VKHIP_CONV_GEMM || d->in_scale))
         return set_error(VKHIP_ERR_UNSUPPORTED, "persistent tile %d runs plain GEMM plans only (no split-K, Winograd or input scale)", tile);
     ConvGeom g = gemm_geom(d, tile, wino);
-    plan->algo = algo;
-    plan->tile = tile;
+    plan->algo     = algo;
+    plan->tile     = tile;
+    plan->reserved = nbi;
     size_t wb  = (size_t) g.Coutp * g.Kp * 2;
     plan->weight_bytes = align256((size_t) g.Coutp * 4) + wb * (wino ? 16 : 1);
     if (split) {
