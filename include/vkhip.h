@@ -226,8 +226,8 @@ int vkhip_conv_forward_stages(const vkhip_conv_desc *d, const vkhip_conv_plan *p
  * GPU (zero at load, left zero by every call); plans with more output tiles are rejected. */
 #define VKHIP_NOALLOC_MAX_TILES 16384
 /* Depthwise conv that also leaves, for a following global average pool, the sum of its stored fp16
- * outputs per (plane, row tile): pool is [N*ceil(C/4)][R] x 4 fp32, R = vkhip_conv_pool_parts
- * (0: the plan's kernel cannot; then use vkhip_conv_forward and vkhip_global_avg_pool). y is
+ * outputs in R parts per plane: pool is [N*ceil(C/4)][R] x 4 fp32, R = vkhip_conv_pool_parts, one part
+ * per row strip or one or more per band of rows (0: the plan's kernel cannot; then use vkhip_conv_forward and vkhip_global_avg_pool). y is
  * exactly what vkhip_conv_forward writes. No counterpart in the reference (its GlobalAveragePool
  * re-reads the conv output, cpu/ops/global_avg_pool.cpp:7-28). */
 int vkhip_conv_pool_parts(const vkhip_conv_desc *d, const vkhip_conv_plan *plan);

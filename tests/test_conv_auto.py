@@ -96,3 +96,16 @@ def test_plans_of_large_maps_cost_no_walk():
                 assert plan_of(V.CONV_GEMM, 33, 0, **c)[0] == 0
             best[n] = min(best[n], (time.perf_counter() - t) / 20)
     assert best[128] < best[1] + 10e-6, best
+
+
+@pytest.mark.parametrize("c,h,w,k,s", [(64, 112, 112, 3, 1), (96, 112, 112, 3, 2), (32, 224, 224, 3, 1), (72, 56, 56, 5, 2), (960, 7, 7, 5, 1)])
+def test_pool_parts_do_not_grow_with_the_row_bands(c, h, w, k, s):
+    """The FC after a depthwise conv adds its parts up one by one: at most 4 bands of a plane (8 past
+    128 rows), each with the 16-window groups that its row can lie in, also for one image, where the
+    conv without pool sums splits into many more."""
+    d = V.ConvDesc(N=1, Cin=c, H=h, W=w, Cout=c, OH=(h - 1) // s + 1, OW=(w - 1) // s + 1, KH=k, KW=k, SH=s, SW=s, PT=k // 2, PL=k // 2, DH=1, DW=1, group=c, act=1)
+    p = V.ConvPlan()
+    assert V.vkhip().vkhip_conv_plan_make(ctypes.byref(d), V.CONV_DEPTHWISE, -1, 0, ctypes.byref(p)) == 0
+    windows = -(-d.OW // (4 if s == 1 else 2))
+    parts = V.vkhip().vkhip_conv_pool_parts(ctypes.byref(d), ctypes.byref(p))
+    assert 0 < parts <= (8 if d.OH > 128 else 4) * ((windows + 14) // 16 + 1)

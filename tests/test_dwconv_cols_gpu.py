@@ -117,7 +117,8 @@ def test_cols_residual_in_place_beside_infinities(gpu, k, s, pooled):
     np.testing.assert_array_equal(from_device_nc4(dy, ys), ref)
 
 
-@pytest.mark.parametrize("shape,k,s", [((3, 22, 14, 14), 3, 1), ((4, 960, 7, 7), 5, 1), ((2, 12, 29, 31), 5, 2), ((1, 8, 40, 9), 3, 2)])
+@pytest.mark.parametrize("shape,k,s", [((3, 22, 14, 14), 3, 1), ((4, 960, 7, 7), 5, 1), ((2, 12, 29, 31), 5, 2), ((1, 8, 40, 9), 3, 2),
+                                       ((2, 8, 20, 112), 3, 1), ((1, 5, 140, 77), 3, 1), ((1, 4, 37, 300), 5, 2)])
 def test_cols_pool_sums(gpu, shape, k, s):
     """The parts of a plane add up to the sum of the stored fp16 outputs: fp32 sums of at most
     H * W values each, so their relative error is below H * W * 2^-24 < 1e-4."""

@@ -1371,7 +1371,7 @@ static int conv_forward_impl(const vkhip_conv_desc *d, const vkhip_conv_plan *pl
         a.pool = (float4v *) pool;
         bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
         DwCols cols;
-        if (plan->tile == 0 && dw_cols_plan(d, cols)) return dw_cols_launch(a, cols, st);
+        if (plan->tile == 0 && dw_cols_plan(d, pool != nullptr, cols)) return dw_cols_launch(a, cols, st);
         DwTile t;
         const int RT = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
         if (unit && d->KH == d->KW && (d->KH == 3 || d->KH == 5) && (d->SH == 1 || d->SH == 2) &&
@@ -1575,7 +1575,7 @@ int vkhip_conv_forward_view_res(const vkhip_conv_desc *d, const vkhip_conv_plan 
 int vkhip_conv_pool_parts(const vkhip_conv_desc *d, const vkhip_conv_plan *plan) {
     if (!d || !plan || plan->algo != VKHIP_CONV_DEPTHWISE || d->in_scale) return 0;
     DwCols cols;
-    if (plan->tile == 0 && dw_cols_plan(d, cols)) return cols.NB * cols.parts;
+    if (plan->tile == 0 && dw_cols_plan(d, true, cols)) return cols.NB * cols.parts;
     const bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
     const int  RT   = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
     DwTile     t;

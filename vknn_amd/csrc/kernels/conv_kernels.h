@@ -2255,7 +2255,7 @@ namespace vkhip {
         int Q;          // columns per channel block: N * NB * XB
         int parts;      // pool sums per (plane, band): the groups that its windows can lie in
     };
-    bool dw_cols_plan(const vkhip_conv_desc *d, DwCols &t);
+    bool dw_cols_plan(const vkhip_conv_desc *d, bool pooled, DwCols &t); // pooled: the split of a launch with pool sums
     int  dw_cols_launch(const DwArgs &a, const DwCols &t, hipStream_t st);
 
 } // namespace vkhip

@@ -242,12 +242,16 @@ namespace vkhip {
     // square 3x3 / 5x5, stride 1 or 2, and taps that stay inside the 8-pixel window.
     // Bands: whole planes while that makes enough waves (2048, two per SIMD), else down to 4 rows
     // (the K - 1 extra input rows of a band are read again by its neighbour).
+    // With pool sums every band adds t.parts of them to what each FC tile after it sums up, 0.15 us each,
+    // where a row less per band saves 0.2 us: 4 bands, 8 past 128 rows. Conv and squeeze-excite of one
+    // image, bands as without the sums (by the wave count) -> 4 or 8: 64 channels 112x112 3x3 27.8 -> 17.0
+    // us, 96 at 112 / 2 3x3 21.5 -> 14.2, 72 at 56 3x3 16.4 -> 14.1, 32 at 224 3x3 63.2 -> 23.3.
     // A 3x3 stride-2 conv whose tensors exceed the last-level cache stays with the strip kernel, which
     // reads them in longer runs: 64 channels 112 -> 56 at batch 128 (257 MB) 49.3 us against 59.1,
     // 56 -> 28 at batch 512 49.8 against 55.3; below (77 MB) 17.3 against 15.3, and the other kernel
     // sizes and strides are level or faster here on both sides (3x3 stride 1, 321 MB: 72.8 / 73.0;
     // 5x5 stride 2, 201 MB: 51.2 / 45.2).
-    bool dw_cols_plan(const vkhip_conv_desc *d, DwCols &t) {
+    bool dw_cols_plan(const vkhip_conv_desc *d, bool pooled, DwCols &t) {
         const int K = d->KH, S = d->SH;
         if (d->DH != 1 || d->DW != 1 || d->KW != K || d->SW != S || (K != 3 && K != 5) || (S != 1 && S != 2)) return false;
         const int DX = S == 1 ? 4 : 2;
@@ -258,7 +262,8 @@ namespace vkhip {
         t.XB = (int) ceil_div(d->OW, DX);
         t.NB = 1;
         auto rows = [&](int nb) { return (int) round_up(ceil_div(d->OH, nb), S); };
-        while (Cb * ceil_div((int64_t) d->N * t.XB * t.NB, 16) < 2048 && rows(t.NB) > 4) ++t.NB;
+        const int most = !pooled ? d->OH : d->OH > 128 ? 8 : 4;
+        while (t.NB < most && Cb * ceil_div((int64_t) d->N * t.XB * t.NB, 16) < 2048 && rows(t.NB) > 4) ++t.NB;
         t.BR = rows(t.NB);
         t.NB = (int) ceil_div(d->OH, t.BR);
         const int64_t Q = (int64_t) d->N * t.XB * t.NB;
