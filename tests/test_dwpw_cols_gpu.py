@@ -59,6 +59,19 @@ def test_cols_pads(gpu, k, s, pads):
     assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
 
 
+# one or two projection fragments x strips of 4, 2 and 1 rows per thread; ragged channels, one chunk
+# and many, a strip of several row groups and one cut off by the last row
+@pytest.mark.parametrize("shape,pads,cout,dw_act,act,res", [((2, 72, 12, 16), (2, 1, 2, 3), 40, 2, 0, True), ((1, 144, 14, 14), (2, 3, 2, 1), 24, 1, 3, False),
+                                                            ((3, 20, 4, 64), (1, 1, 1, 3), 24, 0, 1, False), ((3, 20, 4, 64), (1, 1, 1, 3), 33, 2, 0, True),
+                                                            ((2, 33, 3, 38), (1, 3, 1, 1), 7, 2, 0, False), ((2, 33, 3, 38), (1, 3, 1, 1), 64, 2, 4, False),
+                                                            ((1, 1024, 6, 8), (2, 1, 2, 3), 64, 2, 0, False), ((2, 4, 9, 100), (2, 1, 2, 3), 16, 2, 0, True)])
+def test_ring_kernel_on_odd_left_pads(gpu, shape, pads, cout, dw_act, act, res):
+    """5x5 stride 1 with an odd left pad, the one case that stays on the ring kernel."""
+    got, ref = run(shape, 5, 1, pads, cout, dw_act, act, res)
+    rel, cos = parity(got, ref)
+    assert rel <= 2e-2 and cos >= 0.9999, (rel, cos)
+
+
 @pytest.mark.parametrize("k,s", [(3, 1), (3, 2), (5, 1), (5, 2)])
 @pytest.mark.parametrize("dw_act", [0, 2])
 def test_cols_infinities_stay_in_their_window(gpu, k, s, dw_act):

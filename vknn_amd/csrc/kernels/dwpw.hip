@@ -696,24 +696,21 @@ namespace vkhip {
         return fits();
     }
 
+    // The ring kernel is built for 5x5 stride 1 only: dwpw_cols_kernel takes every other shape it fits.
     typedef void (*RingFn)(DwPwArgs, DwRing);
-    template <int K, int S, int MF, int NS>
+    constexpr int kRingNS = 2; // LDS stages: faster than three on every shape (the third costs a workgroup per CU)
+    template <int MF>
     static RingFn ring_rtt(int rtt) {
         switch (rtt) {
-            case 4: return dwpw_ring_kernel<K, S, MF, 4, NS>;
-            case 2: return dwpw_ring_kernel<K, S, MF, 2, NS>;
-            case 1: return dwpw_ring_kernel<K, S, MF, 1, NS>;
+            case 4: return dwpw_ring_kernel<5, 1, MF, 4, kRingNS>;
+            case 2: return dwpw_ring_kernel<5, 1, MF, 2, kRingNS>;
+            case 1: return dwpw_ring_kernel<5, 1, MF, 1, kRingNS>;
         }
         return nullptr;
     }
-    template <int NS>
-    static RingFn ring_fn_ns(int K, int S, int mf, int rtt) {
-        if (K == 3) {
-            if (S == 1) return mf == 1 ? ring_rtt<3, 1, 1, NS>(rtt) : ring_rtt<3, 1, 2, NS>(rtt);
-            return mf == 1 ? ring_rtt<3, 2, 1, NS>(rtt) : ring_rtt<3, 2, 2, NS>(rtt);
-        }
-        if (S == 1) return mf == 1 ? ring_rtt<5, 1, 1, NS>(rtt) : ring_rtt<5, 1, 2, NS>(rtt);
-        return mf == 1 ? ring_rtt<5, 2, 1, NS>(rtt) : ring_rtt<5, 2, 2, NS>(rtt);
+    static RingFn dwpw_ring_fn(int K, int S, int mf, int rtt) {
+        if (K != 5 || S != 1) return nullptr;
+        return mf == 1 ? ring_rtt<1>(rtt) : ring_rtt<2>(rtt);
     }
 
     // LDS bytes of the ring kernel: NS stages of T KB plus the B chunk
@@ -962,27 +959,25 @@ int vkhip_dwpw_forward(const vkhip_dwpw_desc *d, const void *x, const void *blob
     // VKHIP_DWPW_STRIP=0 keeps the untiled kernel (A/B measurements)
     const char *strip_env = std::getenv("VKHIP_DWPW_STRIP");
     const bool  strip_on  = !(strip_env && strip_env[0] == '0');
-    // VKHIP_DWPW_RING=0 keeps the strip kernel (A/B measurements). Two LDS stages: measured
-    // faster than three on every shape, since the third stage costs a workgroup per CU.
+    // VKHIP_DWPW_RING=0 keeps the strip kernel (A/B measurements)
     const char *ring_env = std::getenv("VKHIP_DWPW_RING");
     const bool  ring_on  = !(ring_env && ring_env[0] == '0');
-    constexpr int kRingNS = 2;
     DwRing rt;
     int    RTT = 0;
     if (ring_on && dwpw_ring_fits(d, g, kRingNS, rt, RTT)) {
         // The column kernel reads the ring kernel's fp16 taps and was faster on all 32 shapes measured (its
         // comment lists some), so the ring is left the 5x5 stride 1 convs with an odd left pad, whose
-        // windows do not fit. VKHIP_DWPW_COLS=0 keeps the ring kernel (A/B measurements).
-        const char *cols_env = std::getenv("VKHIP_DWPW_COLS");
-        DwPwCols    ct;
-        if (!(cols_env && cols_env[0] == '0') && dwpw_cols_plan(d, ct)) return dwpw_cols_launch(a, ct, resolve_stream(s));
+        // windows do not fit: there it beats the strip kernel (240 -> 40 at 28x28 b32 45.3 us against
+        // 63.3, 960 -> 64 at 8x8 b32 58.3 against 88.7).
+        DwPwCols ct;
+        if (dwpw_cols_plan(d, ct)) return dwpw_cols_launch(a, ct, resolve_stream(s));
         rt.x_bytes    = (int) (c.N * g.Eb * c.H * c.W * 8);
         rt.blob_bytes = (int) g.bytes;
         rt.off_dwb    = (int) g.off_dwb;
         rt.off_dww    = (int) g.off_dwh;
         rt.off_pww    = (int) g.off_pww;
         rt.blob       = blob;
-        RingFn fn     = ring_fn_ns<kRingNS>(c.KH, c.SH, (int) g.m_frags, RTT);
+        RingFn fn     = dwpw_ring_fn(c.KH, c.SH, (int) g.m_frags, RTT);
         if (fn) {
             dim3 grid((unsigned) (c.N * ceil_div(c.OH, rt.SR)));
             fn<<<grid, 256, dwpw_ring_lds(rt, kRingNS), resolve_stream(s)>>>(a, rt);

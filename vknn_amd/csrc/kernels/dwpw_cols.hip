@@ -226,7 +226,7 @@ namespace vkhip {
 
     // The column split of a shape that dwpw_ring_fits accepts (square 3x3 / 5x5, stride 1 or 2, no
     // dilation, even width, at most 64 output channels, 31-bit buffer offsets), or false where the taps
-    // of a window's outputs reach past its 8 pixels (5x5 stride 1 and 2 with an odd left pad).
+    // of a window's outputs reach past its 8 pixels (5x5 stride 1 with an odd left pad).
     bool dwpw_cols_plan(const vkhip_dwpw_desc *d, DwPwCols &t) {
         const vkhip_conv_desc &c = d->dw;
         const int     DX = c.SH == 1 ? 4 : 2;
