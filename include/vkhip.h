@@ -172,14 +172,16 @@ typedef struct vkhip_conv_plan {
     int32_t tile;            /* GEMM tile configuration index (see vkhip_conv_tile_count) */
     int32_t ksplit;          /* split-K parts (SPLITK only) */
     int32_t reserved;        /* for reports, not read by forward calls: 3x3 halo tiles, the 1 KB copies
-                              * per channel slot of the largest input band (0 for other tiles) */
+                              * per channel slot of the largest input band; depthwise, the kernel that
+                              * the tile comes to (vkhip_conv_plan_kernel names it); 0 for other plans */
     size_t  weight_bytes;    /* size of the packed weight blob */
     size_t  workspace_bytes; /* device scratch the forward call needs (0 = none) */
 } vkhip_conv_plan;
 
 /* Fill `plan` for `algo` (AUTO picks by shape heuristics). `tile` < 0 picks the default tile; for
  * a depthwise conv `tile` is the number of output rows per strip of the row-tiled kernel (4, 7 or
- * 14; 0 or < 0: chosen by shape, the matrix-core kernel wherever its 8-pixel window holds the taps). */
+ * 14; 0 or < 0: chosen by shape, the matrix-core kernel where its 8-pixel window holds the taps of a
+ * square 3x3 / 5x5 without dilation, except 3x3 stride 2 over more than 160 MiB of tensors). */
 int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, int32_t ksplit, vkhip_conv_plan *plan);
 int vkhip_conv_tile_count(void);
 /* Name of the kernel family a plan launches (e.g. "conv_dma_kernel"; Winograd names its three

@@ -109,3 +109,18 @@ def test_pool_parts_do_not_grow_with_the_row_bands(c, h, w, k, s):
     windows = -(-d.OW // (4 if s == 1 else 2))
     parts = V.vkhip().vkhip_conv_pool_parts(ctypes.byref(d), ctypes.byref(p))
     assert 0 < parts <= (8 if d.OH > 128 else 4) * ((windows + 14) // 16 + 1)
+
+
+@pytest.mark.parametrize("tile,kernel,c", [
+    (-1, "dwconv_cols_kernel", dict(KH=3, KW=3)), (-1, "dwconv_cols_kernel", dict(KH=5, KW=5, PT=2, PL=2)),
+    (7, "dwconv_lds_kernel", dict(KH=3, KW=3)), (907, "dwconv_lds_kernel", dict(KH=3, KW=3, H=7, W=7, OH=7, OW=7)),
+    (-1, "dwconv_lds_kernel", dict(KH=5, KW=5, OH=16, OW=16)),  # left pad 1: the taps leave the window
+    (-1, "dwconv_lds_kernel", dict(N=128, Cin=64, Cout=64, group=64, H=112, W=112, OH=56, OW=56, KH=3, KW=3, SH=2, SW=2)),  # 257 MB
+    (-1, "dwconv_kernel", dict(KH=7, KW=7, PT=3, PL=3)), (7, "dwconv_kernel", dict(KH=7, KW=7, PT=3, PL=3)),
+    (-1, "dwconv_kernel", dict(KH=3, KW=3, DH=2, DW=2, PT=2, PL=2)), (4, "dwconv_kernel", dict(H=6, W=300, OH=6, OW=300, KH=3, KW=3))])
+def test_depthwise_plans_name_the_kernel_they_run(tile, kernel, c):
+    """Reports and profiles take a layer's kernel from its plan, which knows what its tile comes to."""
+    d = V.ConvDesc(**{**dict(N=2, Cin=8, H=18, W=18, Cout=8, OH=18, OW=18, SH=1, SW=1, PT=1, PL=1, DH=1, DW=1, group=8, act=1), **c})
+    p = V.ConvPlan()
+    assert V.vkhip().vkhip_conv_plan_make(ctypes.byref(d), V.CONV_DEPTHWISE, tile, 0, ctypes.byref(p)) == 0
+    assert V.vkhip().vkhip_conv_plan_kernel(ctypes.byref(p)).decode() == kernel

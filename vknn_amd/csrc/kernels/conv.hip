@@ -649,6 +649,20 @@ namespace vkhip {
         return (unsigned) std::max<int64_t>(q, res / q * q);
     }
 
+    // The kernel that runs a depthwise plan's tile, and its split of the work: tile 0 the column kernel
+    // where that applies, else the strip kernel (3x3 / 5x5 of unit dilation whose strip fits LDS), else
+    // the untiled one. RT: rows per strip.
+    enum { DW_UNTILED, DW_STRIPS, DW_COLS };
+    static int dw_route(const vkhip_conv_desc *d, int tile, bool pooled, DwCols &cols, DwTile &t, int &RT) {
+        if (tile == 0 && dw_cols_plan(d, pooled, cols)) return DW_COLS;
+        RT = tile > 0 ? tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
+        const bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
+        return unit && d->KH == d->KW && (d->KH == 3 || d->KH == 5) && (d->SH == 1 || d->SH == 2) &&
+                       dw_tile(d, (int64_t) d->N * ceil_div(d->Cin, 4), RT, std::max(1, tile / 100), t)
+                   ? DW_STRIPS
+                   : DW_UNTILED;
+    }
+
     // ------------------------------------------------------------------ host side: plans
 
     // the kernel of tile `tile` (kTiles), by family
@@ -1095,7 +1109,7 @@ const char *vkhip_conv_plan_kernel(const vkhip_conv_plan *plan) {
     static const char *kinds[] = {"conv_gemm_kernel", "conv_bd_kernel", "conv_dma_kernel", "conv_halo_kernel", "conv_stem_kernel", "conv_thin_kernel"};
     if (!plan) return "?";
     if (plan->algo == VKHIP_CONV_GEMM && plan->tile >= 0 && plan->tile < kNumTiles && kTiles[plan->tile].PERS) return "conv_dma_persist_kernel";
-    if (plan->algo == VKHIP_CONV_DEPTHWISE) return plan->tile ? "dwconv_lds_kernel" : "dwconv_cols_kernel";
+    if (plan->algo == VKHIP_CONV_DEPTHWISE) return plan->reserved == DW_COLS ? "dwconv_cols_kernel" : plan->reserved == DW_STRIPS ? "dwconv_lds_kernel" : "dwconv_kernel";
     if (plan->tile < 0 || plan->tile >= kNumTiles) return "?";
     if (plan->algo == VKHIP_CONV_WINOGRAD) return "wino_input_kernel+conv_gemm_kernel+wino_output_kernel";
     return kinds[kTiles[plan->tile].kind];
@@ -1137,6 +1151,10 @@ int vkhip_conv_plan_make(const vkhip_conv_desc *d, int32_t algo, int32_t tile, i
         plan->algo         = VKHIP_CONV_DEPTHWISE;
         plan->tile         = tile > 0 ? tile : 0;
         plan->weight_bytes = align256((size_t) Cb * 4 * 4) + (size_t) Cb * d->KH * d->KW * 8;
+        DwCols cols;
+        DwTile t;
+        int    RT = 0;
+        plan->reserved     = dw_route(d, plan->tile, false, cols, t, RT);
         return VKHIP_OK;
     }
     if (d->group != 1) return set_error(VKHIP_ERR_UNSUPPORTED, "grouped conv");
@@ -1369,13 +1387,13 @@ static int conv_forward_impl(const vkhip_conv_desc *d, const vkhip_conv_plan *pl
         a.KH = d->KH; a.KW = d->KW; a.SH = d->SH; a.SW = d->SW; a.PT = d->PT; a.PL = d->PL; a.DH = d->DH; a.DW = d->DW;
         a.act = d->act; a.lo = d->act_lo; a.hi = d->act_hi; a.has_res = d->has_res;
         a.pool = (float4v *) pool;
-        bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
+        const bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
         DwCols cols;
-        if (plan->tile == 0 && dw_cols_plan(d, pool != nullptr, cols)) return dw_cols_launch(a, cols, st);
         DwTile t;
-        const int RT = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
-        if (unit && d->KH == d->KW && (d->KH == 3 || d->KH == 5) && (d->SH == 1 || d->SH == 2) &&
-            dw_tile(d, (int64_t) d->N * Cb, RT, std::max(1, plan->tile / 100), t)) {
+        int    RT = 0;
+        const int route = dw_route(d, plan->tile, pool != nullptr, cols, t, RT);
+        if (route == DW_COLS) return dw_cols_launch(a, cols, st);
+        if (route == DW_STRIPS) {
             const bool   pers = plan->tile >= 900;
             const size_t tile_bytes = (size_t) t.PP * t.PS * 8;
             // the pool reduction reuses the tile, or (persistent groups: the halo must survive) follows it
@@ -1575,14 +1593,10 @@ int vkhip_conv_forward_view_res(const vkhip_conv_desc *d, const vkhip_conv_plan 
 int vkhip_conv_pool_parts(const vkhip_conv_desc *d, const vkhip_conv_plan *plan) {
     if (!d || !plan || plan->algo != VKHIP_CONV_DEPTHWISE || d->in_scale) return 0;
     DwCols cols;
-    if (plan->tile == 0 && dw_cols_plan(d, true, cols)) return cols.NB * cols.parts;
-    const bool unit = d->DH == 1 && d->DW == 1 && d->SH == d->SW;
-    const int  RT   = plan->tile > 0 ? plan->tile % 100 : (d->OH % 7 == 0 ? 7 : 4);
-    DwTile     t;
-    if (!(unit && d->KH == d->KW && (d->KH == 3 || d->KH == 5) && (d->SH == 1 || d->SH == 2) &&
-          dw_tile(d, (int64_t) d->N * ceil_div(d->Cin, 4), RT, std::max(1, plan->tile / 100), t)))
-        return 0;
-    return t.row_tiles;
+    DwTile t;
+    int    RT = 0;
+    const int route = dw_route(d, plan->tile, true, cols, t, RT);
+    return route == DW_COLS ? cols.NB * cols.parts : route == DW_STRIPS ? t.row_tiles : 0;
 }
 
 int vkhip_conv_forward_pooled(const vkhip_conv_desc *d, const vkhip_conv_plan *plan, const void *x, const void *blob, const void *res,
