@@ -1500,8 +1500,8 @@ namespace vkhip {
     }
 
     // ------------------------------------------------------------------ 3x3 halo-tile GEMM kernel
-    // Direct 3x3 pad-1 convolution, stride 1 or 2 (the last K stage of a channel count that is not a
-    // multiple of 16*KK is filled with zero slots),
+    // Direct 3x3 pad-1 convolution, stride 1 or 2 (Cin a multiple of 16*KK, or RAG: the last K stage is
+    // filled with zero slots),
     // that reads each input pixel once per workgroup instead of once per tap: the workgroup's BN
     // consecutive output pixels (row-major over n, oy, ox, free to cross image boundaries) need a
     // band of input rows (rows S*oy - 1 .. S*oy + 1 of each output row oy);
@@ -1521,6 +1521,9 @@ namespace vkhip {
     //   pair that holds pixel W-1 also copies the next image row's first pixel into column W, the
     //   right pad; the B fragments of the right-hand taps are zeroed in registers for the output
     //   columns whose right neighbour is that pad.
+    //   RAG: any channel count. The test of each copy costs channel counts that need none 1-5% on most
+    //   tiles (one image, 64 x 128 tile, 256 -> 256 at 14x14 13.5 us without it, 13.9 with; 32 x 256 tile,
+    //   512 -> 512 / 2 at 14x14 24.3 and 25.5), so it is a variant.
     // LDS bytes of a halo workgroup: NS ring stages plus the spare 1 KB that surplus A copies fill
     template <int FM, int WM, int WN, int KK, int NS, int NBI>
     __host__ __device__ constexpr int halo_lds_bytes() {
@@ -1530,7 +1533,7 @@ namespace vkhip {
     // The halo kernel's main loop (everything before its epilogue): the workgroup (m_tile, n0)
     // accumulates its BM x BN tile over K stages ks_begin .. ks_end of split `split` into acc,
     // with the ring in `sm` (halo_lds_bytes).
-    template <int FM, int FN, int WM, int WN, int KK, int NS, int NBI, bool ODD>
+    template <int FM, int FN, int WM, int WN, int KK, int NS, int NBI, bool ODD, bool RAG = false>
     __device__ __forceinline__ void halo_mainloop(const GemmArgs &a, unsigned char *sm, float16v (&acc)[FM][FN], int tid, int lane, int wave,
                                                   int m_tile, int n0, int split) {
         constexpr int NW     = WM * WN;
@@ -1608,9 +1611,9 @@ namespace vkhip {
             for (int r = 0; r < NBW; ++r) {
                 const int c  = r * NW + wave;
                 const int sl = c / NBI;
-                // slots past the last channel block (a channel count that fills no whole stage): zeros
-                const bool     in = ks * SLOTS + sl < a.Cinb; // wave-uniform
-                const unsigned vo = in ? bsrc[c % NBI] : kInvalid;
+                // RAG: slots past the last channel block are zeros (wave-uniform)
+                const bool     in = !RAG || ks * SLOTS + sl < a.Cinb;
+                const unsigned vo = in ? bsrc[c % NBI] : kInvalid; // (a local: the host pass rejects the array element as a builtin operand)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void *) (dst + BOFF + sl * SS + (c % NBI) * 1024),
                                                          16, vo, in ? (unsigned) (ks * SLOTS + sl) * hw8 : 0u, 0, 0);
             }
@@ -1711,7 +1714,7 @@ namespace vkhip {
         }
     }
 
-    template <int FM, int FN, int WM, int WN, int KK, int NS, int NBI, bool ODD = false>
+    template <int FM, int FN, int WM, int WN, int KK, int NS, int NBI, bool ODD, bool RAG>
     __global__ __launch_bounds__(64 * WM * WN, 1) void conv_halo_kernel(GemmArgs a) {
         constexpr int BM = 32 * FM * WM;
         constexpr int BN = 32 * FN * WN;
@@ -1724,7 +1727,7 @@ namespace vkhip {
         const int n0     = (lin / a.m_tiles) * BN;
         const int split  = blockIdx.y;
         float16v  acc[FM][FN];
-        halo_mainloop<FM, FN, WM, WN, KK, NS, NBI, ODD>(a, sm, acc, tid, lane, wave, m_tile, n0, split);
+        halo_mainloop<FM, FN, WM, WN, KK, NS, NBI, ODD, RAG>(a, sm, acc, tid, lane, wave, m_tile, n0, split);
         gemm_epilogue<FM, FN>(a, acc, m_tile * BM + (wave / WN) * 32 * FM, n0 + (wave % WN) * 32 * FN, split, 0, lane,
                               reinterpret_cast<volatile int *>(sm));
     }
@@ -2129,8 +2132,8 @@ namespace vkhip {
     // kind 2: conv_dma_kernel (A and B via LDS DMA; dense B only: 1x1 s1 with an even pixel count
     //         per image, Winograd GEMMs with an even tile count), 2x2 waves of (32FM) x (32FN).
     // kind 3: conv_halo_kernel (3x3 pad-1, stride 1 or 2: input band staged once in LDS for all 9
-    //         taps), KK 16-channel K steps per LDS stage. RC = b: the kernel and geometry of tile b,
-    //         for any channel count (tile b keeps to multiples of 16*KK). Against the best gather tile
+    //         taps), KK 16-channel K steps per LDS stage. RC = b: the geometry of tile b, its
+    //         kernel's RAG variant: any channel count (tile b keeps to multiples of 16*KK). Against the best gather tile
     //         on counts that are not (us): 65 -> 341 at 35x17 b37 39.3 -> 23.7, 333 -> 47 at 15x57 b110
     //         90.7 -> 45.5, 149 -> 46 at 69x18 b24 20.2 -> 11.3, 72 -> 72 at 28x28 b32 17.5 -> 9.9,
     //         201 -> 71 stride 2 at 76x74 b3 19.9 -> 13.9: the gather reads each input pixel 9 times.
