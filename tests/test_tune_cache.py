@@ -216,3 +216,33 @@ def test_warm_start_takes_prepacked_weights_from_cache_file(lib, tmp_path):
     lib.vknn_weight_cache_stats(ctypes.byref(n), ctypes.byref(h), ctypes.byref(m))
     assert h.value == 0 and m.value == convs
     np.testing.assert_array_equal(s5.run(x), y1)
+
+
+@pytest.mark.gpu
+def test_entries_that_never_compared_a_kernel_are_tuned_again(lib):
+    """Picks of a depthwise layer, of a 3x3 over a channel count that fills no whole K stage and of a
+    depthwise + projection pair under the keys of tables from before the matrix-core depthwise, any-channel
+    halo and fused column kernels: the layers are tuned under the keys of the present set; a pick under
+    such a key is taken."""
+    V.require_gpu()
+    buf = ctypes.create_string_buffer(128)
+    lib.vknn_tune_cache_gpu_tag(buf, 128)
+    tag = buf.value + b"/"
+    dw, pair = b"conv_2_144_56_56_144_56_56_3_3_1_1_1_1_1_1_144_0_4", b"dwpw%s_2_144_56_56_56_56_3_3_1_1_1_1_24_1"
+    strip = 4 | (7 + 1) << 8
+    lib.vknn_tune_cache_clear()
+    lib.vknn_tune_cache_put(tag + dw, strip)
+    lib.vknn_tune_cache_put(tag + pair % b"", 1)
+    V.Session("mnv2_block", 2, seed=3, options="tuning=fast;fuse_dwpw=1")
+    assert get(lib, tag + dw + b"_k2") is not None and get(lib, tag + pair % b"2") is not None
+    lib.vknn_tune_cache_put(tag + dw + b"_k2", strip)
+    lib.vknn_tune_cache_put(tag + pair % b"2", 1)
+    s = V.Session("mnv2_block", 2, seed=3, options="tuning=fast;fuse_dwpw=1")
+    assert "split: dw + 1x1" in s.describe()
+    s = V.Session("mnv2_block", 2, seed=3, options="tuning=fast;hip_auto_dwpw=0")
+    assert "depthwise tile=7" in s.describe()
+    lib.vknn_tune_cache_clear()
+    V.Session("conv_tiny", 2, seed=3, options="tuning=fast")
+    ragged = b"conv_2_6_9_9_6_9_9_3_3_1_1_1_1_1_1_1_0_4"
+    assert get(lib, tag + ragged) is None and get(lib, tag + ragged + b"_k2") is not None
+    lib.vknn_tune_cache_clear()

@@ -119,6 +119,13 @@ namespace vknn {
             if (d.in_scale) k += "_xs";
             return k;
         }
+        // Suffix of the cache key of a layer whose candidates a kernel has joined since tables were first
+        // written: an entry from before did not compare that kernel, so it is tuned again. 2: depthwise convs
+        // (the matrix-core kernel) and 3x3s that fill no whole 16-channel K stage (the any-channel halo tiles).
+        static const char *comparedSet(const vkhip_conv_desc &d) {
+            const bool ragged3x3 = d.KH == 3 && d.KW == 3 && d.PT == 1 && d.PL == 1 && d.DH == 1 && d.DW == 1 && d.Cin % 16;
+            return d.group > 1 || ragged3x3 ? "_k2" : "";
+        }
         // (algo, tile, ksplit) <-> one i32 table value: algo in bits 0-7, tile+1 in 8-15, ksplit in 16-23
         static int32_t encodePick(const std::array<int32_t, 3> &p) { return (p[0] & 0xff) | (((p[1] + 1) & 0xff) << 8) | ((p[2] & 0xff) << 16); }
         static std::array<int32_t, 3> decodePick(int32_t v) { return {v & 0xff, ((v >> 8) & 0xff) - 1, (v >> 16) & 0xff}; }
@@ -276,7 +283,7 @@ namespace vknn {
                     build(w, b);
                     return;
                 }
-                const std::string key = keyOf(d, tuning * 4 + wino) + (viewIO ? "_view" : "");
+                const std::string key = keyOf(d, tuning * 4 + wino) + (viewIO ? "_view" : "") + comparedSet(d);
                 tuneKey               = key;
                 int32_t           cached = 0;
                 if (TuneCache::instance().get(key, cached)) {
@@ -560,7 +567,7 @@ namespace vknn {
                 dwc.choosePlan(env, dw_w, dw_b);
                 pwc.choosePlan(env, pw_w, pw_b);
                 mid = std::make_shared<DevBuf>(nc4Bytes({c.N, c.Cin, c.OH, c.OW}));
-                std::string key = gpuTag() + "/dwpw";
+                std::string key = gpuTag() + "/dwpw2"; // 2: the fused kernel with both stages on the matrix cores
                 for (int v: {c.N, c.Cin, c.H, c.W, c.OH, c.OW, c.KH, c.KW, c.SH, c.SW, c.PT, c.PL, d.Cout, d.has_res})
                     key += "_" + std::to_string(v);
                 int32_t cached = 0;
