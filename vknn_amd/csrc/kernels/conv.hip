@@ -989,10 +989,12 @@ namespace vkhip {
     // The plan AUTO takes for a dense 1x1 (pad 0) or 3x3 (pad 1) layer at stride 1 or 2: the cheapest one
     // predicted among the plans that accept it; first layers (at most 4 channels) take the thin kernel.
     // Leaves `algo` at AUTO where none of them applies (other kernels, pads, dilations, an input scale):
-    // the gather tiles then. Over those layers the picks are 3-4% slower than the best measured plan of
+    // the gather tiles then. Over the fitted layers the picks are 3-4% slower than the best measured plan of
     // each layer and, in the geometric mean, 1.49x (1x1), 1.10x (1x1 stride 2), 1.73x (3x3) and 1.35x (3x3
-    // stride 2) faster than the gather tiles, the only ones AUTO knew before; on 300 other layers 1.54x. 256 -> 1024 at 14x14 b64 with a residual: 42.8 -> 21.2 us; 3x3 256 -> 256 there: 45.2 -> 21.8.
-    // First layers: 7x7 / 2 3 -> 64 at 224 b64 185 -> 39.7 us, 3x3 / 2 3 -> 16 at 640 b16 146 -> 22.5.
+    // stride 2) faster than the gather tiles, the only ones AUTO knew before; on 140 other layers 1.54x,
+    // 1.18x, 1.89x and 1.42x, the worst pick 3% slower. 256 -> 1024 at 14x14 b64 with a residual: 40.9 ->
+    // 21.1 us; 3x3 256 -> 256 there: 43.2 -> 20.3. First layers: 45 of them 1.51x, the worst 3% slower;
+    // 7x7 / 2 3 -> 64 at 224 b64 185 -> 39.7 us, 3x3 / 2 3 -> 16 at 640 b16 146 -> 22.5.
     // Splits: only where the output is small and the reduction deep, and never a workspace that the
     // allocation-free entry point could not hold.
     static void auto_pick(const vkhip_conv_desc *d, int32_t &algo, int32_t &tile, int32_t &ksplit) {
