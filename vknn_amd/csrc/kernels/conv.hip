@@ -1026,7 +1026,7 @@ namespace vkhip {
                     if (tab[i].tile == p.tile && (tab[i].split != 0) == split) best = (one ? 0.9f : 0.95f) * auto_cost(d, tab[i], std::max(1, p.ksplit));
         }
         for (int i = 0; i < n; ++i) {
-            // a 3x3 over a multiple of 16 channels takes the tile that the any-channel tile shares its kernel with
+            // a 3x3 over a multiple of 16 channels takes the tile of the same geometry that tests no channels
             const int rc = kTiles[tab[i].tile].RC, t = rc && d->Cin % 16 == 0 ? rc : tab[i].tile;
             for (int ks: {1, 2, 3, 4, 6, 8, 12, 16}) {
                 if ((ks > 1) != (tab[i].split != 0) || (ks > 1 && !may_split)) continue;
